@@ -79,10 +79,9 @@ struct ckd_ctx {
     uint32_t lsFog0 = 0;
     uint32_t *lsQuadH = nullptr;
     uint4 *lsQuadC = nullptr;
-    // ckd_landscape_draw's work queue of march ranges: four control words
-    // and one 64-bit state word per column of a launch's frames
-    uint32_t *lsQueue = nullptr;
-    unsigned long long *lsState = nullptr;
+    // the fog table in 16-bit lanes and the span lengths' divisors
+    uint2 *lsFogLanes = nullptr;
+    uint16_t *lsSpanDiv = nullptr;
 
     // tunnelscape maps (Tunnelscape_Create)
     uint8_t *tsHeight = nullptr;

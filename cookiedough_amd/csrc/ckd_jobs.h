@@ -16,7 +16,7 @@ struct SdfJob {
     float invH;         // 1 / H, rounded to nearest
 };
 
-// voxel request: 64-column blocks, one lane per column
+// voxel request: blocks of voxel_block_cols() columns
 struct VoxJob {
     uint32_t *dst;
     uint32_t W, H;

@@ -181,16 +181,23 @@ CKD_DEV void ckd_span_setup_drawn(CkdSpan &s, uint32_t A, uint32_t B, uint32_t l
     }
 }
 
+// packus_epi16 of two 16-bit lanes: v_sat_pk_u8_i16 clamps each (signed) to
+// [0, 255] and packs them into the low two bytes
+CKD_DEV uint32_t ckd_sat_pk_u8(uint32_t lanes)
+{
+    uint32_t r;
+    asm("v_sat_pk_u8_i16 %0, %1" : "=v"(r) : "v"(lanes));
+    return r;
+}
+
 // one span pixel: v = acc>>16 (logical); packus_epi32 keeps v (<= 65535);
-// packus_epi16 maps v > 32767 to 0 and clamps to 255.  v > 32767 is a
-// negative acc, so the channel is byte 2 of acc clamped (signed) to
-// [0, 0xffffff]: one v_med3_i32 per channel, two byte permutes per pixel.
+// packus_epi16 maps v > 32767 (a negative lane) to 0 and clamps to 255: the
+// high halves of two accumulators per v_sat_pk_u8_i16, three byte permutes
 CKD_DEV uint32_t ckd_span_pixel(const uint32_t acc[4])
 {
-    uint32_t m[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) m[k] = (uint32_t)min(max((int32_t)acc[k], 0), 0xffffff);
-    return ckd_perm(m[1], m[0], 0x0c0c0602u) | ckd_perm(m[3], m[2], 0x06020c0cu);
+    const uint32_t lo = ckd_sat_pk_u8(ckd_perm(acc[1], acc[0], 0x07060302u));
+    const uint32_t hi = ckd_sat_pk_u8(ckd_perm(acc[3], acc[2], 0x07060302u));
+    return ckd_perm(hi, lo, 0x05040100u);
 }
 
 // ---- 2007 box blur helpers --------------------------------------------

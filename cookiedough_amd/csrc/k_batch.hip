@@ -21,7 +21,9 @@ ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t 
                                  int shading, unsigned long long *stepCount, bool helper,
                                  bool alone);
 void voxel_job_geometry(VoxJob &J, unsigned W, unsigned H, const ckd_landscape_cam &c);
-ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, uint32_t totalBlocks);
+unsigned voxel_block_cols(size_t columns);
+ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, uint32_t totalBlocks,
+                                 unsigned blockCols);
 void tunnel_job_geometry(TunJob &J, uint32_t *dst, uint32_t *tmp, const int32_t *grid, unsigned W,
                          unsigned H, int radius);
 uint32_t tunnel_vblocks(unsigned W, unsigned H, int seg);
@@ -69,6 +71,7 @@ struct Plan {
     size_t oSdf = 256, oVox = 0, oTun = 0;
     int nSdf = 0, nVox = 0, nTun = 0;
     uint32_t chunks = 0, voxBlocks = 0, tunRows = 0, tunV = 0;
+    unsigned voxCols = 0; // columns per voxel block
     unsigned tunMaxW = 0;
     unsigned tunMaxE = 0;
 };
@@ -126,7 +129,10 @@ void make_plan(const ckd_tuning &T, const ckd_request *requests, unsigned n, uin
     std::vector<VoxJob> vox;
     std::vector<TunJob> tun;
     const uint32_t chunk = (uint32_t)T.sdfChunk;
-    size_t off = 0;
+    size_t off = 0, voxColumns = 0;
+    for (unsigned i = 0; i < n; ++i)
+        if (requests[i].effect == CKD_FX_VOXEL) voxColumns += requests[i].W;
+    P.voxCols = ckd::voxel_block_cols(voxColumns);
     for (unsigned i = 0; i < n; ++i) {
         const ckd_request &r = requests[i];
         if (r.effect == CKD_FX_SDF) {
@@ -145,7 +151,7 @@ void make_plan(const ckd_tuning &T, const ckd_request *requests, unsigned n, uin
             J.dst = r.dst;
             ckd::voxel_job_geometry(J, r.W, r.H, r.vcam);
             J.blockBase = P.voxBlocks;
-            P.voxBlocks += (r.W + 63) / 64;
+            P.voxBlocks += (r.W + P.voxCols - 1) / P.voxCols;
             vox.push_back(J);
         } else {
             TunJob J;
@@ -205,7 +211,7 @@ ckd_status launch_plan(ckd_ctx *ctx, const Plan &P, unsigned char *dev, const ck
         ckd::StreamSwap swap(ctx, fork ? ctx->aux : ctx->stream);
         if (P.nVox > 0) {
             s = ckd::launch_landscape_jobs(ctx, reinterpret_cast<const VoxJob *>(dev + P.oVox),
-                                           P.nVox, P.voxBlocks);
+                                           P.nVox, P.voxBlocks, P.voxCols);
             if (s != CKD_OK) return s;
         }
         if (P.nTun > 0 && !split) {

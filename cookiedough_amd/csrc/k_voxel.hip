@@ -1,11 +1,13 @@
 // k_voxel.hip -- voxel landscape columns (code/landscape.cpp) and the
 // tunnelscape rows (code/tunnelscape.cpp).
 //
-// One lane per column (rows for tunnelscape) marches the reference's 512
-// front-to-back steps and draws the visible spans with the exact
-// cspanISSE16 arithmetic.  The memset32 of the fog colour is fused: after
-// the march every lane fills the part of its column no span reached, so
-// each pixel is written exactly once.
+// Both march the reference's 512 front-to-back steps per column (row for
+// tunnelscape) and draw the visible spans with the exact cspanISSE16
+// arithmetic: the landscape spreads a column's steps over a block (the
+// highest row drawn so far, the only value that carries, is a prefix
+// minimum), the tunnelscape runs one lane per row.  The memset32 of the fog
+// colour is fused: after the march the part of a column no span reached is
+// filled, so each pixel is written exactly once.
 #include "ckd_internal.h"
 #include "ckd_pixel.h"
 #include "ckd_jobs.h"
@@ -17,6 +19,8 @@
 namespace {
 
 constexpr unsigned kMapAnd = 1023, kMapShift = 10, kRayLength = 512;
+// span lengths with a divisor of their own: 65536 / n is 0 from 65537 on
+constexpr unsigned kSpanDivs = 65538;
 // march steps whose texels are fetched ahead of the step being drawn
 constexpr int kLsAhead = 4;
 
@@ -26,8 +30,7 @@ struct LsFrame {
 };
 
 // frames per launch, their parameters passed by value: 160 keeps the
-// kernel's arguments inside the 4 KiB limit, and one launch of that many
-// 1280-column frames is 3200 waves, enough to fill every SIMD
+// kernel's arguments inside the 4 KiB limit
 constexpr int kLsFramesPerLaunch = 160;
 
 struct LsLaunch {
@@ -35,45 +38,7 @@ struct LsLaunch {
     int mapScale;
     LsFrame f[kLsFramesPerLaunch];
 };
-static_assert(sizeof(LsLaunch) + 64 <= 4096, "k_landscape's arguments fit 4 KiB");
-
-// bsamp32_16 (code/bilinear.h:58-83) followed by _mm_subs_epu16 of the fog
-// colour (code/landscape.cpp:83): the interpolation runs on two channels per
-// register (B,R and G,A in 16-bit lanes, exact as in ckd_bilerp32) and the
-// saturating subtract is one packed u16 subtract per pair
-CKD_DEV uint32_t ls_bilerp_fog(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, uint32_t fu,
-                               uint32_t fv, uint32_t fogBR, uint32_t fogGA)
-{
-    const uint32_t M = 0x00ff00ffu;
-    const ckd_u16x2 f = ckd_splat16(fu), g = ckd_splat16(fv);
-    const ckd_u16x2 nf = (unsigned short)256 - f, ng = (unsigned short)256 - g;
-    const ckd_u16x2 br = ckd_lerp2x(ckd_lerp2x(ckd_u16x2_of(p0 & M), ckd_u16x2_of(p1 & M), nf, f),
-                                    ckd_lerp2x(ckd_u16x2_of(p2 & M), ckd_u16x2_of(p3 & M), nf, f),
-                                    ng, g);
-    const ckd_u16x2 ga =
-        ckd_lerp2x(ckd_lerp2x(ckd_u16x2_of(ckd_odd_bytes(p0)), ckd_u16x2_of(ckd_odd_bytes(p1)), nf, f),
-                   ckd_lerp2x(ckd_u16x2_of(ckd_odd_bytes(p2)), ckd_u16x2_of(ckd_odd_bytes(p3)), nf, f),
-                   ng, g);
-    const ckd_u16x2 sbr = __builtin_elementwise_sub_sat(br, ckd_u16x2_of(fogBR));
-    const ckd_u16x2 sga = __builtin_elementwise_sub_sat(ga, ckd_u16x2_of(fogGA));
-    return ckd_u32_of(sbr) | (ckd_u32_of(sga) << 8);
-}
-
-// (255 - bsamp8(quad)) << 16 (code/bilinear.h:34-53, code/landscape.cpp:
-// 76-86) for a height quad h4 holding (u,v), (u+1,v), (u,v+1), (u+1,v+1) in
-// bytes 0..3: both horizontal lerps in the 16-bit lanes of (h0,h2) and
-// (h1,h3), the vertical one as the sum of the lanes of (s01*(256-fv),
-// s23*fv).  Every intermediate lies in [0, 65280], as in the scalar form.
-CKD_DEV uint32_t ls_height_num(uint32_t h4, uint32_t fu, uint32_t fv)
-{
-    const ckd_u16x2 f = ckd_splat16(fu), nf = (unsigned short)256 - f;
-    const ckd_u16x2 s = ckd_lerp2x(ckd_u16x2_of(ckd_perm(0u, h4, 0x0c020c00u)),  // h0, h2
-                                   ckd_u16x2_of(ckd_perm(0u, h4, 0x0c030c01u)),  // h1, h3
-                                   nf, f);                                       // s01, s23
-    const ckd_u16x2 p = s * ckd_u16x2{(unsigned short)(256u - fv), (unsigned short)fv};
-    const uint32_t sum = (uint32_t)p[0] + (uint32_t)p[1];
-    return 0xff0000u - ckd_perm(0u, sum, 0x0c010c0cu); // (255 - (sum >> 8)) << 16
-}
+static_assert(sizeof(LsLaunch) + 128 <= 4096, "the kernel's arguments fit 4 KiB");
 
 // exact floor(num/den) for num < 2^24 and 0 < den < 2^24 with a quotient
 // below 2^22: num * rcp(den) is then within 0.5 of num/den, so the estimate
@@ -141,235 +106,355 @@ __global__ __launch_bounds__(256) void k_ls_quads(const uint8_t *__restrict__ hm
     quadC[i] = make_uint4(cmap[u + v0], cmap[u1 + v0], cmap[u + v1], cmap[u1 + v1]);
 }
 
-// vscape_ray (code/landscape.cpp:56-107) for column iRay of one frame, march
-// steps [s0, s1).  drawnIn() gives the highest row the steps before s0 drew
-// (H when s0 is 0); it is called once the first texels are in flight.  The
-// fused memset32(fog[0]) for the rows no span reached runs when s1 ends the
-// march.  Returns the highest row drawn after step s1 - 1.
-template <typename DrawnIn>
-CKD_DEV int ls_column(global_u32 *__restrict__ col, unsigned W, unsigned H, unsigned iRay,
-                      float rayY, float colScale, float halfW, int mapScale, float X1, float Y1,
-                      float viewCos, float viewSin, int mapTilt,
-                      const uint32_t *__restrict__ quadH, const uint4 *__restrict__ quadC,
-                      const uint32_t *__restrict__ fog, unsigned s0, unsigned s1, DrawnIn drawnIn)
+// the fog table as the colour blend subtracts it, fog[k]'s B,R and G,A in the
+// high bytes of 16-bit lanes, and floor(65536 / n) mod 2^16 for a span of n
+// rows (0 for n = 0 and beyond 65535: nothing there reads its high bit)
+__global__ __launch_bounds__(256) void k_ls_tables(const uint32_t *__restrict__ fog, uint2 *__restrict__ fogLanes,
+                                                   uint16_t *__restrict__ spanDiv)
 {
-    int dX, dY, fpFishMul;
-    ls_setup(rayY, colScale, halfW, X1, Y1, viewCos, viewSin, iRay, dX, dY, fpFishMul);
-    int curX = (int)(X1 * 256.f), curY = (int)(Y1 * 256.f);
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 256) fogLanes[i] = make_uint2((fog[i] << 8) & 0xff00ff00u, fog[i] & 0xff00ff00u);
+    if (i < kSpanDivs) spanDiv[i] = i ? (uint16_t)(65536u / i) : (uint16_t)0;
+}
 
-    // The march is software-pipelined: the texels of the next kLsAhead steps
-    // are in flight while a step draws its span (only curX/curY carry from
-    // step to step, and every fetch is masked into the maps, so fetches past
-    // the last step are harmless).
-    struct Texels {
-        uint32_t h4, fu, fv;
-        uint4 c;
-    };
-    auto fetch = [&](Texels &t) {
-        curX += dX;
-        curY += dY;
-        const unsigned i = ((((unsigned)(curY >> 8)) & kMapAnd) << kMapShift) |
-                           (((unsigned)(curX >> 8)) & kMapAnd);
-        t.fu = (uint32_t)curX & 0xff;
-        t.fv = (uint32_t)curY & 0xff;
-        t.h4 = quadH[i];
-        t.c = quadC[i];
-    };
-    // a step's projected row and fogged colour (f = fog[iStep >> 1], den =
-    // fpFishMul * (iStep + 1))
-    auto sample = [&](const Texels &t, uint32_t f, uint32_t den, int &hgt, uint32_t &color) {
-        color = ls_bilerp_fog(t.c.x, t.c.y, t.c.z, t.c.w, t.fu, t.fv, f & 0x00ff00ffu, (f >> 8) & 0x00ff00ffu);
+// ---- vscape_ray (code/landscape.cpp:56-107) over a block ---------------------
+//
+// A column's 512 steps depend on each other only through the highest row
+// drawn so far, a running minimum.  A block takes kCols columns, thread
+// (segment, column) kSteps consecutive steps of one of them:
+//   1  the projected rows of its steps: heights only
+//   2  a prefix minimum over the segments gives every step the row D drawn
+//      before it; the steps that draw (row < D) go packed into a list in LDS
+//   3  one lane per listed span: its two colours, its set-up, its pixels
+//   4  the rows no span reached take the fog colour
+// One lane per column, the form before, left a 1280-column frame 20 waves on
+// 1024 SIMDs and fetched and blended a colour at every step; about 30% of the
+// steps draw (155 of 512 at 1280x720), the rest are hidden behind nearer ones.
+// What bounds it: VALU issue, 4 cycles an instruction; 27 for a step's row, 10
+// for its place in the list, about 105 for a span and 12 for each of its
+// pixels.  Measured, one lane per column -> now: 1 frame of 1280x720 172 -> 8.5
+// us, 30 of 1366x768 184 -> 73 us, 90 of them 289 -> 198 us, 150 of 1280x720
+// 391 -> 289 us.
+//
+// The list is ordered by (wave, step of the run, lane), so that neighbouring
+// lanes take the same step of neighbouring columns: their texels share cache
+// lines and their pixels rows.  Blocks that follow one another go to one XCD
+// (ls_block_of): the parts of a 128-byte line that neighbouring blocks write
+// then meet in its L2 (150 frames 329 -> 296 us).
+template <int kCols, int kSteps> constexpr int kLsThreads = kCols * (int)kRayLength / kSteps;
 
-        // ((255-h)<<16) / (fpFishMul*(iStep+1)) is an unsigned division
-        // fpFishMul <= 256 and iStep < 512: 24-bit multiplies are exact;
-        // q < 2^17 (fpFishMul >= 191 at every width) and mapScale < 2^11
-        const uint32_t q = udiv24(ls_height_num(t.h4, t.fu, t.fv), den);
-        hgt = ((int)ckd_mul_u24(q, (uint32_t)mapScale) >> 8) + mapTilt;
-    };
+// list entries per column: frames of the bench's landscape draw 140 to 170
+// spans a column.  A block with more goes through its list in rounds.
+constexpr int kLsListPerCol = 192;
 
-    int lastHeight = (int)H, lastDrawn;
-    uint32_t lastColor;
-    if (s0 == 0) {
-        lastColor = quadC[(((unsigned)(curX >> 8)) & kMapAnd) | ((((unsigned)(curY >> 8)) & kMapAnd) << kMapShift)].x;
-    } else {
-        // the march's state after step s0 - 1: that step's row and colour
-        // (s0 - 1 additions of dX wrap as one multiply-add does)
-        curX = (int)((uint32_t)curX + (uint32_t)dX * (s0 - 1));
-        curY = (int)((uint32_t)curY + (uint32_t)dY * (s0 - 1));
-        Texels t;
-        fetch(t);
-        sample(t, fog[(s0 - 1) >> 1], ckd_mul_u24((uint32_t)fpFishMul, s0), lastHeight, lastColor);
+// a drawn span: step i of column c, rows [hgt, D), length rows to the row of
+// step i - 1.  hgt < D <= H <= 2160; length < 2^20 (a projected row is below
+// 23071 * W >> 8 plus the tilt)
+CKD_DEV uint2 ls_span(uint32_t c, uint32_t i, int hgt, int D, int prev)
+{
+    return make_uint2((uint32_t)hgt | ((uint32_t)D << 12) | (c << 24), i | ((uint32_t)(prev - hgt) << 9));
+}
+
+// the projected row of a step (code/landscape.cpp:76-86) from a height quad
+// h4 holding (u,v), (u+1,v), (u,v+1), (u+1,v+1) in bytes 0..3: bsamp8
+// (code/bilinear.h:34-53), both horizontal lerps in the 16-bit lanes of (h0,h2)
+// and (h1,h3), the vertical one a dot product; then ((255 - h) << 16) / den *
+// mapScale >> 8 plus the tilt (tilt8 = 256 * tilt).  den = fish * (step + 1) <=
+// 2^17 as a float; fish >= 8 keeps the quotient below 2^22, so that num *
+// rcp(den) is within 0.5 of num / den, the estimate truncated is the quotient
+// or one less and one upward correction fixes it; the remainder, an integer
+// below 2^18, is exact from one FMA.  Checked on the host over every (num,
+// den) with den = fish * (step + 1) and fish >= 4, the reciprocal rounded to
+// nearest and one ulp off either way.
+CKD_DEV int ls_row(uint32_t h4, uint32_t x, uint32_t y, float denF, uint32_t mapScale, uint32_t tilt8)
+{
+    // both lanes fu, then 256 - fu
+    const ckd_u16x2 f = ckd_u16x2_of(ckd_perm(0u, x, 0x0c000c00u)), nf = (unsigned short)256 - f;
+    const ckd_u16x2 s = ckd_lerp2x(ckd_u16x2_of(ckd_perm(0u, h4, 0x0c020c00u)),
+                                   ckd_u16x2_of(ckd_perm(0u, h4, 0x0c030c01u)), nf, f);
+    // lanes (256 - fv, fv) = fv * 65535 + 256
+    const ckd_u16x2 g = ckd_u16x2_of(__umul24(y & 0xffu, 0xffffu) + 256u);
+    const uint32_t sum = __builtin_amdgcn_udot2(s, g, 0u, false);
+    // (255 - (sum >> 8)) << 16, exact in FP32
+    const float num = __builtin_fmaf((float)((sum >> 8) & 0xffu), -65536.f, 16711680.f);
+    const float q = truncf(__builtin_fmaf(num, __builtin_amdgcn_rcpf(denF), -0.5f));
+    const uint32_t n = (uint32_t)(int32_t)q + (__builtin_fmaf(-q, denF, num) >= denF ? 1u : 0u);
+    return (int)(__umul24(n, mapScale) + tilt8) >> 8;
+}
+
+// bsamp32_16 (code/bilinear.h:58-83) of a texel quad at (x, y) followed by
+// _mm_subs_epu16 of the fog colour (code/landscape.cpp:83), channels in the
+// 16-bit lanes of br and ga.  The fog (f, k_ls_tables) is subtracted before
+// the blend's last >> 8: v - 256 * fog, saturated at 0, then >> 8 is
+// max((v >> 8) - fog, 0).
+CKD_DEV void ls_color(const uint4 &q, uint32_t x, uint32_t y, uint2 f, ckd_u16x2 &br, ckd_u16x2 &ga)
+{
+    const uint32_t M = 0x00ff00ffu;
+    const ckd_u16x2 u = ckd_u16x2_of(ckd_perm(0u, x, 0x0c000c00u)), v = ckd_u16x2_of(ckd_perm(0u, y, 0x0c000c00u));
+    const ckd_u16x2 nu = (unsigned short)256 - u, nv = (unsigned short)256 - v;
+    const ckd_u16x2 b = ckd_lerp2x(ckd_u16x2_of(q.x & M), ckd_u16x2_of(q.y & M), nu, u) * nv +
+                        ckd_lerp2x(ckd_u16x2_of(q.z & M), ckd_u16x2_of(q.w & M), nu, u) * v;
+    const ckd_u16x2 g = ckd_lerp2x(ckd_u16x2_of(ckd_odd_bytes(q.x)), ckd_u16x2_of(ckd_odd_bytes(q.y)), nu, u) * nv +
+                        ckd_lerp2x(ckd_u16x2_of(ckd_odd_bytes(q.z)), ckd_u16x2_of(ckd_odd_bytes(q.w)), nu, u) * v;
+    br = __builtin_elementwise_sub_sat(b, ckd_u16x2_of(f.x)) >> (unsigned short)8;
+    ga = __builtin_elementwise_sub_sat(g, ckd_u16x2_of(f.y)) >> (unsigned short)8;
+}
+
+// int16 lane kHi of a times the low int16 of b, plus c
+template <bool kHi> CKD_DEV uint32_t ls_mad16(uint32_t a, uint32_t b, uint32_t c)
+{
+    uint32_t r;
+    if constexpr (kHi)
+        asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    else
+        asm("v_mad_i32_i16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+template <bool kHi> CKD_DEV uint32_t ls_mul16(uint32_t a, uint32_t b)
+{
+    uint32_t r;
+    if constexpr (kHi)
+        asm("v_mad_i32_i16 %0, %1, %2, 0 op_sel:[1,0,0,0]" : "=v"(r) : "v"(a), "v"(b));
+    else
+        asm("v_mad_i32_i16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// ckd_span_setup_drawn from colours in 16-bit lanes (A the span's first, B
+// its last), the low 16 bits of the divisor and the pre-step length: the
+// deltas as two packed subtracts, each product with the divisor or the
+// pre-step (their low 16 bits, signed) one v_mad_i32_i16
+CKD_DEV void ls_span_setup(CkdSpan &s, ckd_u16x2 Abr, ckd_u16x2 Aga, ckd_u16x2 Bbr, ckd_u16x2 Bga,
+                           uint32_t divisor, uint32_t pre)
+{
+    const uint32_t m = ckd_mul_u24_v(divisor, pre);
+    const uint32_t br = ckd_u32_of(Bbr - Abr), ga = ckd_u32_of(Bga - Aga);
+    const uint32_t a = ckd_u32_of(Abr), g = ckd_u32_of(Aga);
+    s.step[0] = ls_mul16<false>(br, divisor);
+    s.step[1] = ls_mul16<false>(ga, divisor);
+    s.step[2] = ls_mul16<true>(br, divisor);
+    s.step[3] = ls_mul16<true>(ga, divisor);
+    s.acc[0] = ls_mad16<false>(br, m, a << 16);
+    s.acc[1] = g << 16;
+    s.acc[2] = ls_mad16<true>(br, m, a & 0xffff0000u);
+    s.acc[3] = g & 0xffff0000u;
+}
+
+// the parameters every column of a frame shares
+struct LsView {
+    unsigned W, H;
+    float rayY, colScale, halfW;
+    int mapScale;
+    LsFrame f;
+};
+
+struct LsMaps {
+    const uint32_t *quadH;
+    const uint4 *quadC;
+    const uint2 *fogLanes;
+    const uint16_t *spanDiv;
+    uint32_t sky; // fog[0]
+};
+
+template <int kCols, int kSteps>
+CKD_DEV void ls_block(global_u32 *__restrict__ dst, const LsView &V, const LsMaps &M, unsigned col0)
+{
+    constexpr int kThreads = kLsThreads<kCols, kSteps>, kWaves = kThreads / 64;
+    static_assert(kThreads % 64 == 0 && kThreads <= 1024 && kCols <= 32, "whole waves of whole step runs");
+    constexpr int kBatch = kSteps < 8 ? kSteps : 8, kList = kCols * kLsListPerCol;
+    const unsigned W = V.W, H = V.H;
+    __shared__ uint2 spans[kList];
+    __shared__ int rayDX[kCols], rayDY[kCols], rayFish[kCols], top[kCols];
+    __shared__ int waveMin[kWaves][kCols], waveLast[kWaves][kCols];
+    __shared__ uint32_t waveCount[kWaves];
+    __shared__ uint2 fogS[kRayLength / 2];
+    const unsigned t = threadIdx.x, lane = t & 63;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const unsigned c = t % kCols, seg = t / kCols;
+    const bool valid = col0 + c < W;
+    for (unsigned k = t; k < kRayLength / 2; k += kThreads) fogS[k] = M.fogLanes[k];
+    if (t < kCols) {
+        int dX, dY, fish;
+        ls_setup(V.rayY, V.colScale, V.halfW, V.f.X1, V.f.Y1, V.f.viewCos, V.f.viewSin, min(col0 + t, W - 1), dX,
+                 dY, fish);
+        rayDX[t] = dX;
+        rayDY[t] = dY;
+        rayFish[t] = fish;
     }
+    __syncthreads();
+    const int X0 = (int)(V.f.X1 * 256.f), Y0 = (int)(V.f.Y1 * 256.f);
 
-    // den = fpFishMul * (iStep + 1), one add per step (below 2^17)
-    uint32_t den = ckd_mul_u24((uint32_t)fpFishMul, s0);
-    auto step = [&](const Texels &t, uint32_t f) {
-        den += (uint32_t)fpFishMul;
-        int hgt;
-        uint32_t color;
-        sample(t, f, den, hgt, color);
-        if (hgt < lastDrawn) {
-            const uint32_t drawLength = (uint32_t)(lastDrawn - hgt);
-            const uint32_t length = (uint32_t)(lastHeight - hgt);
-            CkdSpan sp;
-            ckd_span_setup_drawn(sp, color, lastColor, length, drawLength, udiv24(65536u, length));
-            // hgt < H <= 2160 and W <= 4096: the row offset fits 24 bits
-            global_u32 *p = col + ckd_mul_u24((uint32_t)hgt, W);
-            for (uint32_t k = 0; k < drawLength; ++k) {
-                *p = ckd_span_pixel(sp.acc);
-                p += W;
+    // 1: the rows of steps seg * kSteps .. + kSteps - 1 (positions wrap as the
+    // march's running additions do; |dX|, |dY| <= 256)
+    int row[kSteps];
+    {
+        const int dX = rayDX[c], dY = rayDY[c];
+        const float fish = (float)rayFish[c];
+        const int first = (int)(seg * kSteps);
+        uint32_t x = (uint32_t)X0 + (uint32_t)__mul24(dX, first), y = (uint32_t)Y0 + (uint32_t)__mul24(dY, first);
+        float den = fish * (float)first;
+        const uint32_t tilt8 = (uint32_t)V.f.mapTilt << 8;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) sp.acc[c] += sp.step[c];
+        for (int s0 = 0; s0 < kSteps; s0 += kBatch) {
+            uint32_t h4[kBatch], xs[kBatch], ys[kBatch];
+#pragma unroll
+            for (int s = 0; s < kBatch; ++s) {
+                x += (uint32_t)dX;
+                y += (uint32_t)dY;
+                xs[s] = x;
+                ys[s] = y;
+                const uint32_t at = ((y << 4) & (kMapAnd << (kMapShift + 2))) | ((x >> 6) & (kMapAnd << 2));
+                h4[s] = *(const uint32_t *)((const char *)M.quadH + at);
             }
-            lastDrawn = hgt;
-        }
-        lastHeight = hgt;
-        lastColor = color;
-    };
-    // two register sets, A and B, take turns: a set is refilled only after
-    // it has been consumed, so each fetched set lands in the registers its
-    // consumer reads and the loop carries no copies of values in flight
-    // s0 and s1 are multiples of 2 * kLsAhead = 8, so a group's eight fog
-    // words fog[iStep/2 .. iStep/2 + 3] are one aligned 16-byte load
-    static_assert(kRayLength % (2 * kLsAhead) == 0 && 2 * kLsAhead == 8, "the march runs in whole groups");
-    Texels A[kLsAhead], B[kLsAhead];
 #pragma unroll
-    for (int k = 0; k < kLsAhead; ++k) fetch(A[k]);
-    lastDrawn = drawnIn();
-    for (unsigned iStep = s0; iStep < s1; iStep += 2 * kLsAhead) {
-        const uint4 fg = *reinterpret_cast<const uint4 *>(fog + (iStep >> 1));
-        const uint32_t f8[4] = {fg.x, fg.y, fg.z, fg.w};
+            for (int s = 0; s < kBatch; ++s) {
+                den += fish;
+                row[s0 + s] = ls_row(h4[s], xs[s], ys[s], den, (uint32_t)V.mapScale, tilt8);
+            }
+        }
+    }
+
+    // 2: the row drawn before each step
+    int lo = row[0];
 #pragma unroll
-        for (int k = 0; k < kLsAhead; ++k) {
-            fetch(B[k]);
-            step(A[k], f8[k >> 1]);
-        }
+    for (int s = 1; s < kSteps; ++s) lo = min(lo, row[s]);
 #pragma unroll
-        for (int k = 0; k < kLsAhead; ++k) {
-            fetch(A[k]);
-            step(B[k], f8[(kLsAhead + k) >> 1]);
+    for (unsigned o = kCols; o < 64; o <<= 1) {
+        const int v = __shfl_up(lo, o, 64);
+        if (lane >= o) lo = min(lo, v);
+    }
+    if (lane >= 64 - kCols) {
+        waveMin[wave][c] = lo;
+        waveLast[wave][c] = row[kSteps - 1];
+    }
+    int D = __shfl_up(lo, kCols, 64), prev = __shfl_up(row[kSteps - 1], kCols, 64);
+    __syncthreads();
+    if (lane < kCols) {
+        D = (int)H;
+        prev = wave ? waveLast[wave - 1][c] : (int)H;
+    }
+    D = min(D, (int)H);
+    for (unsigned w = 0; w < wave; ++w) D = min(D, waveMin[w][c]);
+    // a column past the right edge draws nothing
+    const int D0 = valid ? D : INT_MIN;
+    D = D0;
+    uint32_t n = 0;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        n += (uint32_t)__popcll(__ballot(row[s] < D));
+        D = min(D, row[s]);
+    }
+    if (seg == kRayLength / kSteps - 1) top[c] = D;
+    if (lane == 0) waveCount[wave] = n;
+    __syncthreads();
+    uint32_t base0 = 0, total = 0;
+#pragma unroll
+    for (unsigned w = 0; w < kWaves; ++w) {
+        const uint32_t k = __builtin_amdgcn_readfirstlane(waveCount[w]);
+        base0 += w < wave ? k : 0u;
+        total += k;
+    }
+
+    // 4: the rows above every span
+    if (valid) {
+        const int rows = top[c];
+        for (int y = (int)seg; y < rows; y += kThreads / kCols) dst[(size_t)y * W + col0 + c] = M.sky;
+    }
+
+    // the spans kList at a time (nearly always one round)
+    for (uint32_t r0 = 0; r0 < total; r0 += kList) {
+        if (r0) __syncthreads();
+        D = D0;
+        uint32_t base = base0 - r0;
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            const bool vis = row[s] < D;
+            const uint64_t m = __ballot(vis);
+            const uint32_t at = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            if (vis && at < (uint32_t)kList)
+                spans[at] = ls_span(c, seg * kSteps + s, row[s], D, s ? row[s - 1] : prev);
+            base += (uint32_t)__popcll(m);
+            D = min(D, row[s]);
+        }
+        __syncthreads();
+
+        // 3: the spans
+        const uint32_t cnt = min(total - r0, (uint32_t)kList);
+        for (uint32_t k = t; k < cnt; k += kThreads) {
+            const uint2 e = spans[k];
+            const uint32_t hgt = e.x & 0xfffu, drawn = (e.x >> 12) & 0xfffu, sc = e.x >> 24;
+            const uint32_t i = e.y & 0x1ffu, length = e.y >> 9;
+            const int dX = rayDX[sc], dY = rayDY[sc];
+            // the positions of steps i - 1 and i; before step 0 the colour is
+            // the unfogged texel under the origin
+            const uint32_t px = (uint32_t)X0 + (uint32_t)__mul24(dX, (int)i),
+                           py = (uint32_t)Y0 + (uint32_t)__mul24(dY, (int)i);
+            const uint32_t x = px + (uint32_t)dX, y = py + (uint32_t)dY;
+            auto quad = [&M](uint32_t X, uint32_t Y) {
+                const uint32_t at = ((Y << 6) & (kMapAnd << (kMapShift + 4))) | ((X >> 4) & (kMapAnd << 4));
+                return *(const uint4 *)((const char *)M.quadC + at);
+            };
+            const uint4 q0 = quad(px, py), q1 = quad(x, y);
+            const uint2 f0 = fogS[i ? (i - 1) >> 1 : 0], f1 = fogS[i >> 1];
+            const uint32_t divisor = M.spanDiv[min(length, kSpanDivs - 1)];
+            ckd_u16x2 lastBR, lastGA, br, ga;
+            ls_color(q0, px, py, f0, lastBR, lastGA);
+            if (i == 0) {
+                lastBR = ckd_u16x2_of(q0.x & 0x00ff00ffu);
+                lastGA = ckd_u16x2_of(ckd_odd_bytes(q0.x));
+            }
+            ls_color(q1, x, y, f1, br, ga);
+            const uint32_t drawLength = drawn - hgt;
+            CkdSpan sp;
+            ls_span_setup(sp, br, ga, lastBR, lastGA, divisor, length - drawLength);
+            // hgt < H <= 2160 and W <= 4096: pixel offsets fit 24 bits
+            uint32_t at = ckd_mul_u24(hgt, W) + col0 + sc;
+            for (uint32_t j = 0; j < drawLength; ++j) {
+                dst[at] = ckd_span_pixel(sp.acc);
+                at += W;
+#pragma unroll
+                for (int ch = 0; ch < 4; ++ch) sp.acc[ch] += sp.step[ch];
+            }
         }
     }
-    if (s1 == kRayLength) {
-        const uint32_t sky = fog[0];
-        for (int y = 0; y < lastDrawn; ++y) col[(size_t)y * W] = sky;
-    }
-    return lastDrawn;
 }
 
-__global__ __launch_bounds__(64) void k_landscape(uint32_t *__restrict__ dst, unsigned W,
-                                                  unsigned H, const uint32_t *__restrict__ quadH,
-                                                  const uint4 *__restrict__ quadC,
-                                                  const uint32_t *__restrict__ fog, LsLaunch P)
+// the unit a block takes: blocks go to the 8 XCDs in turn, units of one XCD
+// follow one another (the grid is units rounded up to a multiple of 8)
+CKD_DEV unsigned ls_block_of(unsigned units)
 {
-    const unsigned iRay = blockIdx.x * 64 + threadIdx.x;
-    if (iRay >= W) return;
-    const LsFrame &F = P.f[blockIdx.y];
-    ls_column((global_u32 *)(dst + (size_t)blockIdx.y * W * H + iRay), W, H, iRay, P.rayY, P.colScale, P.halfW,
-              P.mapScale, F.X1, F.Y1, F.viewCos, F.viewSin, F.mapTilt, quadH, quadC, fog, 0, kRayLength,
-              [H] { return (int)H; });
+    return (blockIdx.x & 7) * ((units + 7) / 8) + (blockIdx.x >> 3);
+}
+unsigned ls_grid(unsigned units) { return (units + 7) / 8 * 8; }
+
+template <int kCols, int kSteps>
+__global__ __launch_bounds__((kLsThreads<kCols, kSteps>)) void k_landscape(uint32_t *__restrict__ dst, unsigned W,
+                                                                          unsigned H, LsMaps M, LsLaunch P,
+                                                                          unsigned groupsPerFrame, unsigned units)
+{
+    const unsigned u = ls_block_of(units);
+    if (u >= units) return;
+    const unsigned f = u / groupsPerFrame, g = u - f * groupsPerFrame;
+    const LsView V{W, H, P.rayY, P.colScale, P.halfW, P.mapScale, P.f[f]};
+    ls_block<kCols, kSteps>((global_u32 *)(dst + (size_t)f * W * H), V, M, g * kCols);
 }
 
-// ---- the march split into step ranges, dequeued ---------------------------
-//
-// A launch of many frames has nGroups waves of 64 columns; when that is not
-// close to a multiple of the SIMD count, the SIMDs that hold one wave more
-// than the others set the launch time (120 frames of 1280 columns: 2400
-// waves on 1024 SIMDs take as long as 3072).  Split each column's march into 2^c
-// ranges of 512 >> c steps: unit u = k * nGroups + g is range k of group g.
-// Persistent waves take units from a counter in that order.  Range k > 0
-// needs only one value from range k - 1: the highest row drawn so far.  Range
-// k - 1 publishes it per column, tagged (epoch, k), in a 64-bit state word;
-// range k reads it (after its first texels are in flight) and waits while
-// the tag is not there yet.  Range k - 1 was taken earlier, by a wave that
-// runs, and depends only on ranges taken before it, so every wait ends; the
-// wait is also bounded, and a wait that runs out counts in ctl[3] and
-// carries on from row H.
-//
-// ctl: [0] next unit, [1] epoch, [2] waves finished, [3] waits that ran out.
-// The last wave to finish resets [0] and [2] and moves the epoch on, so the
-// next launch starts from a clean queue and tags of this one never match it.
-constexpr int kLsMaxChunkLog2 = 3;
-constexpr unsigned kLsWaitLimit = 1u << 18; // polls, with a sleep between them
-constexpr size_t kLsStateWords = (size_t)kLsFramesPerLaunch * 4096;
-
-CKD_DEV int ls_wait_drawn(const unsigned long long *w, unsigned long long want, int H,
-                          uint32_t *timeouts)
+// every voxel request of a batch in one launch: unit -> job by binary search
+template <int kCols, int kSteps>
+__global__ __launch_bounds__((kLsThreads<kCols, kSteps>)) void k_landscape_jobs(const VoxJob *__restrict__ jobs,
+                                                                               int nJobs, LsMaps M, unsigned units)
 {
-    unsigned long long v = 0;
-    bool ready = false;
-    for (unsigned spin = 0; spin < kLsWaitLimit; ++spin) {
-        if (!ready) {
-            v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ready = (v >> 16) == want;
-        }
-        if (__ballot(!ready) == 0) return (int)(v & 0xffffu);
-        __builtin_amdgcn_s_sleep(2);
-    }
-    if (!ready) atomicAdd(timeouts, 1u);
-    return ready ? (int)(v & 0xffffu) : H;
+    const unsigned u = ls_block_of(units);
+    if (u >= units) return;
+    const VoxJob &J = jobs[ckd_find_job(jobs, nJobs, u, &VoxJob::blockBase)];
+    const LsView V{J.W, J.H, J.rayY, J.colScale, J.halfW, J.mapScale,
+                   LsFrame{J.X1, J.Y1, J.viewCos, J.viewSin, J.mapTilt}};
+    ls_block<kCols, kSteps>((global_u32 *)J.dst, V, M, (u - J.blockBase) * kCols);
 }
 
-__global__ __launch_bounds__(64) void k_landscape_queue(uint32_t *__restrict__ dst, unsigned W,
-                                                        unsigned H, const uint32_t *__restrict__ quadH,
-                                                        const uint4 *__restrict__ quadC,
-                                                        const uint32_t *__restrict__ fog, LsLaunch P,
-                                                        unsigned groupsPerFrame, unsigned nGroups,
-                                                        unsigned chunkLog2, unsigned nWaves,
-                                                        uint32_t *__restrict__ ctl,
-                                                        unsigned long long *__restrict__ state)
+LsMaps ls_maps(const ckd_ctx *ctx)
 {
-    const unsigned lane = threadIdx.x;
-    const uint32_t epoch =
-        __builtin_amdgcn_readfirstlane(__hip_atomic_load(&ctl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    const unsigned steps = kRayLength >> chunkLog2, nChunks = 1u << chunkLog2;
-    const unsigned nUnits = nGroups << chunkLog2;
-    for (;;) {
-        uint32_t u = 0;
-        if (lane == 0) u = atomicAdd(&ctl[0], 1u);
-        u = __builtin_amdgcn_readfirstlane(u);
-        if (u >= nUnits) break;
-        const unsigned k = u / nGroups, g = u - k * nGroups;
-        const unsigned f = g / groupsPerFrame;
-        const unsigned iRay = (g - f * groupsPerFrame) * 64 + lane;
-        if (iRay < W) {
-            const LsFrame &F = P.f[f];
-            unsigned long long *w = state + (size_t)f * W + iRay;
-            const unsigned long long want = ((unsigned long long)epoch << 16) | k;
-            const int drawn = ls_column(
-                (global_u32 *)(dst + (size_t)f * W * H + iRay), W, H, iRay, P.rayY, P.colScale, P.halfW,
-                P.mapScale, F.X1, F.Y1, F.viewCos, F.viewSin, F.mapTilt, quadH, quadC, fog, k * steps,
-                (k + 1) * steps, [&] { return k == 0 ? (int)H : ls_wait_drawn(w, want, (int)H, &ctl[3]); });
-            if (k + 1 < nChunks)
-                __hip_atomic_store(w, ((unsigned long long)epoch << 32) | ((unsigned long long)(k + 1) << 16) |
-                                          (unsigned)drawn,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    // relaxed: a wave's last dequeue returned before this increment was
-    // issued, so the last wave to count sees every dequeue done (an
-    // acquire-release here would write back and invalidate the L2 in every
-    // wave, while frames are being written)
-    if (lane == 0 &&
-        __hip_atomic_fetch_add(&ctl[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nWaves - 1) {
-        __hip_atomic_store(&ctl[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&ctl[2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&ctl[1], epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// every voxel request of a batch in one launch: block -> job by binary search
-__global__ __launch_bounds__(64) void k_landscape_jobs(const VoxJob *__restrict__ jobs, int nJobs,
-                                                       const uint32_t *__restrict__ quadH,
-                                                       const uint4 *__restrict__ quadC,
-                                                       const uint32_t *__restrict__ fog)
-{
-    const int j = ckd_find_job(jobs, nJobs, blockIdx.x, &VoxJob::blockBase);
-    const VoxJob &J = jobs[j];
-    const unsigned iRay = (blockIdx.x - J.blockBase) * 64 + threadIdx.x;
-    if (iRay >= J.W) return;
-    ls_column((global_u32 *)(J.dst + iRay), J.W, J.H, iRay, J.rayY, J.colScale, J.halfW, J.mapScale, J.X1, J.Y1,
-              J.viewCos, J.viewSin, J.mapTilt, quadH, quadC, fog, 0, kRayLength, [&J] { return (int)J.H; });
+    return LsMaps{ctx->lsQuadH, ctx->lsQuadC, ctx->lsFogLanes, ctx->lsSpanDiv, ctx->lsFog0};
 }
 
 // ---- tunnelscape ---------------------------------------------------------
@@ -513,14 +598,28 @@ void voxel_job_geometry(VoxJob &J, unsigned W, unsigned H, const ckd_landscape_c
     J.mapTilt = scale_rows(c.mapTilt, H);
 }
 
-ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, uint32_t totalBlocks)
+// Columns per block of a launch of `columns` columns in all.  Narrow blocks
+// split a small launch finer; wide ones share texels and output lines between
+// their columns.  Measured with 4, 8 and 16 columns: 320 columns 5.1, 6.7, 9.2
+// us; 1280 8.5, 8.4, 11.8; 2560 14.0, 15.1, 15.2; 12 800 32, 29, 31; 41 000 87,
+// 75, 75; 123 000 250, 204, 200; 192 000 395, 312, 294 us.
+unsigned voxel_block_cols(size_t columns) { return columns <= 4096 ? 4 : columns <= 49152 ? 8 : 16; }
+
+ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, uint32_t totalBlocks,
+                                 unsigned blockCols)
 {
     if (totalBlocks == 0) return CKD_OK;
     if (!ctx->lsHeight)
         return fail(CKD_ESTATE, "voxel requests need the landscape maps (ckd_landscape_create)");
     KernelTimer kt(ctx, CKD_KT_LANDSCAPE);
-    k_landscape_jobs<<<totalBlocks, 64, 0, ctx->stream>>>(jobs, nJobs, ctx->lsQuadH, ctx->lsQuadC,
-                                                          ctx->lsFog);
+    const LsMaps M = ls_maps(ctx);
+    const unsigned grid = ls_grid(totalBlocks);
+    if (blockCols == 4)
+        k_landscape_jobs<4, 4><<<grid, kLsThreads<4, 4>, 0, ctx->stream>>>(jobs, nJobs, M, totalBlocks);
+    else if (blockCols == 8)
+        k_landscape_jobs<8, 8><<<grid, kLsThreads<8, 8>, 0, ctx->stream>>>(jobs, nJobs, M, totalBlocks);
+    else
+        k_landscape_jobs<16, 16><<<grid, kLsThreads<16, 16>, 0, ctx->stream>>>(jobs, nJobs, M, totalBlocks);
     return check_launch("landscape jobs");
 }
 
@@ -543,19 +642,13 @@ ckd_status ckd_landscape_create(ckd_ctx *ctx, const uint8_t *heightMap, const ui
     if ((!ctx->lsQuadH && ckd::dev_alloc(&ctx->lsQuadH, kTexels * 4) != hipSuccess) ||
         (!ctx->lsQuadC && ckd::dev_alloc(&ctx->lsQuadC, kTexels * 16) != hipSuccess))
         return ckd::fail(CKD_ENOMEM, "ckd_landscape_create: hipMalloc of the texel quads failed");
-    if (!ctx->lsQueue) {
-        if (ckd::dev_alloc(&ctx->lsQueue, 4 * sizeof(uint32_t)) != hipSuccess)
-            return ckd::fail(CKD_ENOMEM, "ckd_landscape_create: hipMalloc of the work queue failed");
-        CKD_HIP(hipMemsetAsync(ctx->lsQueue, 0, 4 * sizeof(uint32_t), ctx->stream));
-    }
-    if (!ctx->lsState) {
-        if (ckd::dev_alloc(&ctx->lsState, kLsStateWords * sizeof(unsigned long long)) != hipSuccess)
-            return ckd::fail(CKD_ENOMEM, "ckd_landscape_create: hipMalloc of the queue's state failed");
-        CKD_HIP(hipMemsetAsync(ctx->lsState, 0, kLsStateWords * sizeof(unsigned long long), ctx->stream));
-    }
+    if ((!ctx->lsFogLanes && ckd::dev_alloc(&ctx->lsFogLanes, 256 * sizeof(uint2)) != hipSuccess) ||
+        (!ctx->lsSpanDiv && ckd::dev_alloc(&ctx->lsSpanDiv, kSpanDivs * sizeof(uint16_t)) != hipSuccess))
+        return ckd::fail(CKD_ENOMEM, "ckd_landscape_create: hipMalloc of the span tables failed");
+    k_ls_tables<<<ckd_div_up(kSpanDivs, 256), 256, 0, ctx->stream>>>(ctx->lsFog, ctx->lsFogLanes, ctx->lsSpanDiv);
     k_ls_quads<<<kTexels / 256, 256, 0, ctx->stream>>>(ctx->lsHeight, ctx->lsColor, ctx->lsQuadH,
                                                        ctx->lsQuadC);
-    s = ckd::check_launch("landscape quads");
+    s = ckd::check_launch("landscape quads and tables");
     if (s == CKD_OK) CKD_HIP(hipStreamSynchronize(ctx->stream));
     return s;
 }
@@ -586,27 +679,16 @@ ckd_status ckd_landscape_draw(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigned 
             const ckd_landscape_cam &c = cams[f0 + k];
             P.f[k] = LsFrame{c.X1, c.Y1, c.viewCos, c.viewSin, scale_rows(c.mapTilt, H)};
         }
-        const unsigned groupsPerFrame = ckd_div_up(W, 64), nGroups = groupsPerFrame * n;
-        const unsigned simds = 4u * (unsigned)ctx->cuCount;
-        const int chunkLog2 = __builtin_ctz((unsigned)ctx->tuning.voxelChunks);
-        // one wave per group puts ceil(nGroups / simds) waves on the busiest
-        // SIMDs; the work queue pays when that is well above the average
-        const unsigned busiest = ckd_div_up(nGroups, simds);
-        const bool uneven = nGroups > simds && (double)nGroups < 0.9 * (double)busiest * simds;
+        const unsigned cols = ckd::voxel_block_cols((size_t)W * n);
+        const unsigned groupsPerFrame = ckd_div_up(W, cols), units = groupsPerFrame * n, grid = ls_grid(units);
+        uint32_t *out = dst + (size_t)f0 * W * H;
         ckd::KernelTimer kt(ctx, CKD_KT_LANDSCAPE);
-        if (chunkLog2 > 0 && uneven) {
-            // the march ranges through the work queue
-            static_assert(kLsMaxChunkLog2 == 3, "voxelChunks is at most 8");
-            const unsigned nUnits = nGroups << chunkLog2;
-            const unsigned nWaves = std::min(nUnits, simds * (unsigned)ctx->tuning.voxelWavesPerSIMD);
-            k_landscape_queue<<<nWaves, 64, 0, ctx->stream>>>(
-                dst + (size_t)f0 * W * H, W, H, ctx->lsQuadH, ctx->lsQuadC, ctx->lsFog, P, groupsPerFrame,
-                nGroups, (unsigned)chunkLog2, nWaves, ctx->lsQueue, ctx->lsState);
-        } else {
-            dim3 grid(groupsPerFrame, n);
-            k_landscape<<<grid, 64, 0, ctx->stream>>>(dst + (size_t)f0 * W * H, W, H, ctx->lsQuadH,
-                                                      ctx->lsQuadC, ctx->lsFog, P);
-        }
+        if (cols == 4)
+            k_landscape<4, 4><<<grid, kLsThreads<4, 4>, 0, ctx->stream>>>(out, W, H, ls_maps(ctx), P, groupsPerFrame, units);
+        else if (cols == 8)
+            k_landscape<8, 8><<<grid, kLsThreads<8, 8>, 0, ctx->stream>>>(out, W, H, ls_maps(ctx), P, groupsPerFrame, units);
+        else
+            k_landscape<16, 16><<<grid, kLsThreads<16, 16>, 0, ctx->stream>>>(out, W, H, ls_maps(ctx), P, groupsPerFrame, units);
         ckd_status s = ckd::check_launch("landscape");
         if (s != CKD_OK) return s;
     }
