@@ -3,9 +3,9 @@
 //
 // Both march the reference's 512 front-to-back steps per column (row for
 // tunnelscape) and draw the visible spans with the exact cspanISSE16
-// arithmetic: the landscape spreads a column's steps over a block (the
-// highest row drawn so far, the only value that carries, is a prefix
-// minimum), the tunnelscape runs one lane per row.  The memset32 of the fog
+// arithmetic.  The highest row drawn so far, the only value that carries from
+// step to step, is a prefix minimum, so the steps are spread over the lanes
+// of a block (landscape) or a wave (tunnelscape).  The memset32 of the fog
 // colour is fused: after the march the part of a column no span reached is
 // filled, so each pixel is written exactly once.
 #include "ckd_internal.h"
@@ -14,15 +14,12 @@
 
 #include <algorithm>
 #include <cstring>
-#include <vector>
 
 namespace {
 
 constexpr unsigned kMapAnd = 1023, kMapShift = 10, kRayLength = 512;
 // span lengths with a divisor of their own: 65536 / n is 0 from 65537 on
 constexpr unsigned kSpanDivs = 65538;
-// march steps whose texels are fetched ahead of the step being drawn
-constexpr int kLsAhead = 4;
 
 struct LsFrame {
     float X1, Y1, viewCos, viewSin;
@@ -461,97 +458,151 @@ LsMaps ls_maps(const ckd_ctx *ctx)
 
 constexpr unsigned kTsAnd = 2047, kTsShift = 11;
 
-// tscape_ray (code/tunnelscape.cpp:44-100), lane per output row.  The
-// caller guarantees map heights <= 159, so every height is positive.
+// tscape_ray (code/tunnelscape.cpp:44-100), one wave per output row: lane l
+// takes steps 8l .. 8l + 7, a prefix minimum over the lanes gives every step
+// the height D drawn before it, the steps that draw (height < D) go into a
+// list in LDS in step order, then one lane draws one span of it: neighbouring
+// lanes read neighbouring texels and write neighbouring pixels.  The caller
+// guarantees map heights <= 159, so every height is positive.
+// One lane per row, the form before, left a 720-row frame 12 waves; what
+// bounds this one is a row's chain of latencies: 1280x720 351 -> 14.8 us.
+constexpr int kTsSteps = (int)kRayLength / 64;
+
+// a step's height from its bilinear map height h (code/tunnelscape.cpp:75-84):
+// ((159 - h) << 8) / 0.28125 truncated, over the step's number, times 160 >>
+// 8, plus 120.  0.28125 is 9/32: the FP32 quotient of the exact 8192 m / 9 (m
+// = 159 - h) lies within 1/64 of it and its fraction is a multiple of 1/9, so
+// both truncations together are floor(8192 m / (9 n)).  num < 2^21 and den <=
+// 4608: the estimate num * rcp(den) - 0.5 truncated is the quotient or one less
+// (checked on the host over every (m, n)).
+CKD_DEV int ts_height(uint32_t h, uint32_t n)
+{
+    const uint32_t q = udiv24((159u - h) << 13, 9u * n);
+    return (int)(__umul24(q, 160u) >> 8) + 120;
+}
+
 __global__ __launch_bounds__(64) void k_tunnelscape(uint32_t *__restrict__ dst, unsigned W,
                                                     unsigned H, const uint8_t *__restrict__ hmap,
                                                     const uint32_t *__restrict__ cmap,
                                                     const uint32_t *__restrict__ fog,
                                                     float mapStepX, float fromXAdd, int fpFromY,
-                                                    int dX, int dY, float kMapViewLenScale)
+                                                    int dX, int dY)
 {
-    const unsigned iRay = blockIdx.x * 64 + threadIdx.x;
-    if (iRay >= H) return;
-    uint32_t *row = dst + (size_t)iRay * W;
-    int curX, curY = fpFromY;
+    __shared__ uint2 spans[kRayLength];
+    const unsigned lane = threadIdx.x, iRay = blockIdx.x;
+    global_u32 *row = (global_u32 *)(dst + (size_t)iRay * W);
+    uint32_t X0, Y0 = (uint32_t)fpFromY;
     {
 #pragma clang fp contract(off)
         const float mapX = (float)iRay * mapStepX;
         const float fromX = mapX + fromXAdd;
-        curX = (int)(fromX * 256.f);
+        X0 = (uint32_t)(int)(fromX * 256.f);
     }
-    int lastHeight = (int)W, lastDrawn = (int)W;
-    uint32_t lastColor =
-        cmap[(((unsigned)(curX >> 8)) & kTsAnd) | ((((unsigned)(curY >> 8)) & kTsAnd) << kTsShift)];
-    unsigned written = 0;
-    // pipelined as in ls_column: the texels of the next kLsAhead steps are in
-    // flight while a step draws its span (fetches are masked into the maps)
-    struct Texels {
-        uint32_t h[4], c[4], fu, fv;
+    // texel indices of the four neighbours of a position
+    auto corners = [](uint32_t X, uint32_t Y, uint32_t (&at)[4]) {
+        const uint32_t u0 = (X >> 8) & kTsAnd, u1 = ((X >> 8) + 1) & kTsAnd;
+        const uint32_t v0 = ((Y >> 8) & kTsAnd) << kTsShift, v1 = (((Y >> 8) + 1) & kTsAnd) << kTsShift;
+        at[0] = u0 + v0;
+        at[1] = u1 + v0;
+        at[2] = u0 + v1;
+        at[3] = u1 + v1;
     };
-    auto fetch = [&](Texels &t) {
-        curX += dX;
-        curY += dY;
-        const unsigned u0 = ((unsigned)(curX >> 8)) & kTsAnd;
-        const unsigned u1 = ((unsigned)(curX >> 8) + 1) & kTsAnd;
-        const unsigned v0 = (((unsigned)(curY >> 8)) & kTsAnd) << kTsShift;
-        const unsigned v1 = (((unsigned)(curY >> 8) + 1) & kTsAnd) << kTsShift;
-        t.fu = (uint32_t)curX & 0xff;
-        t.fv = (uint32_t)curY & 0xff;
-        t.h[0] = hmap[u0 + v0];
-        t.h[1] = hmap[u1 + v0];
-        t.h[2] = hmap[u0 + v1];
-        t.h[3] = hmap[u1 + v1];
-        t.c[0] = cmap[u0 + v0];
-        t.c[1] = cmap[u1 + v0];
-        t.c[2] = cmap[u0 + v1];
-        t.c[3] = cmap[u1 + v1];
-    };
-    auto step = [&](unsigned iStep, const Texels &t) {
-        const uint32_t h = ckd_bilerp8(t.h[0], t.h[1], t.h[2], t.h[3], t.fu, t.fv);
-        uint32_t color = ckd_bilerp32(t.c[0], t.c[1], t.c[2], t.c[3], t.fu, t.fv);
-        color = ckd_subs_u8x4(color, fog[iStep >> 1]);
 
-        int height = 255 - (int)h - 96;
-        height <<= 8;
-        height = (int)((float)height / kMapViewLenScale);
-        height = (int)((unsigned)height / (iStep + 1));
-        height *= 160;
-        height >>= 8;
-        height += 120;
-
-        if (height < lastDrawn) {
-            const uint32_t drawLength = (uint32_t)(lastDrawn - height);
-            CkdSpan s;
-            ckd_span_setup(s, color, lastColor, (uint32_t)(lastHeight - height), drawLength);
-            for (uint32_t k = 0; k < drawLength; ++k) {
-                row[written + k] = ckd_span_pixel(s.acc);
+    // the heights of this lane's steps
+    const uint32_t first = lane * kTsSteps;
+    int height[kTsSteps];
+    {
+        uint32_t h[kTsSteps][4], x = X0 + (uint32_t)dX * first, y = Y0 + (uint32_t)dY * first;
+        uint32_t fu[kTsSteps], fv[kTsSteps];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) s.acc[c] += s.step[c];
-            }
-            written += drawLength;
-            lastDrawn = height;
-        }
-        lastHeight = height;
-        lastColor = color;
-    };
-    Texels A[kLsAhead], B[kLsAhead];
+        for (int s = 0; s < kTsSteps; ++s) {
+            x += (uint32_t)dX;
+            y += (uint32_t)dY;
+            fu[s] = x & 0xff;
+            fv[s] = y & 0xff;
+            uint32_t at[4];
+            corners(x, y, at);
 #pragma unroll
-    for (int k = 0; k < kLsAhead; ++k) fetch(A[k]);
-    for (unsigned iStep = 0; iStep < kRayLength; iStep += 2 * kLsAhead) {
-#pragma unroll
-        for (int k = 0; k < kLsAhead; ++k) {
-            fetch(B[k]);
-            step(iStep + k, A[k]);
+            for (int k = 0; k < 4; ++k) h[s][k] = hmap[at[k]];
         }
 #pragma unroll
-        for (int k = 0; k < kLsAhead; ++k) {
-            fetch(A[k]);
-            step(iStep + kLsAhead + k, B[k]);
+        for (int s = 0; s < kTsSteps; ++s)
+            height[s] = ts_height(ckd_bilerp8(h[s][0], h[s][1], h[s][2], h[s][3], fu[s], fv[s]), first + s + 1);
+    }
+
+    // the height drawn before each step, the spans in step order
+    int lo = height[0];
+#pragma unroll
+    for (int s = 1; s < kTsSteps; ++s) lo = min(lo, height[s]);
+#pragma unroll
+    for (unsigned o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(lo, o, 64);
+        if (lane >= o) lo = min(lo, v);
+    }
+    int D = __shfl_up(lo, 1, 64), prev = __shfl_up(height[kTsSteps - 1], 1, 64);
+    if (lane == 0) D = prev = (int)W;
+    D = min(D, (int)W);
+    const int top = min(__shfl(lo, 63, 64), (int)W);
+    const int D0 = D;
+    uint32_t n = 0;
+#pragma unroll
+    for (int s = 0; s < kTsSteps; ++s) {
+        n += height[s] < D ? 1u : 0u;
+        D = min(D, height[s]);
+    }
+    uint32_t at = n;
+#pragma unroll
+    for (unsigned o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(at, o, 64);
+        if (lane >= o) at += v;
+    }
+    const uint32_t total = __shfl(at, 63, 64);
+    at -= n;
+    D = D0;
+#pragma unroll
+    for (int s = 0; s < kTsSteps; ++s) {
+        if (height[s] < D) {
+            // height < D <= 4096; the distance to the previous step's height
+            // is below 2^17
+            spans[at++] = make_uint2((uint32_t)height[s] | ((uint32_t)D << 12),
+                                     (first + s) | ((uint32_t)((s ? height[s - 1] : prev) - height[s]) << 9));
+            D = height[s];
+        }
+    }
+    __syncthreads();
+
+    // the spans: pixels W - D .. W - height - 1 of the row
+    for (uint32_t k = lane; k < total; k += 64) {
+        const uint2 e = spans[k];
+        const uint32_t hgt = e.x & 0xfffu, drawn = e.x >> 12, i = e.y & 0x1ffu, length = e.y >> 9;
+        // the positions of steps i - 1 and i; before step 0 the colour is the
+        // unfogged texel under the origin
+        const uint32_t px = X0 + (uint32_t)dX * i, py = Y0 + (uint32_t)dY * i;
+        const uint32_t x = px + (uint32_t)dX, y = py + (uint32_t)dY;
+        uint32_t a0[4], a1[4], c0[4], c1[4];
+        corners(px, py, a0);
+        corners(x, y, a1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c0[j] = cmap[a0[j]];
+            c1[j] = cmap[a1[j]];
+        }
+        const uint32_t f0 = fog[i ? (i - 1) >> 1 : 0], f1 = fog[i >> 1];
+        uint32_t lastColor = ckd_subs_u8x4(ckd_bilerp32(c0[0], c0[1], c0[2], c0[3], px & 0xff, py & 0xff), f0);
+        if (i == 0) lastColor = c0[0];
+        const uint32_t color = ckd_subs_u8x4(ckd_bilerp32(c1[0], c1[1], c1[2], c1[3], x & 0xff, y & 0xff), f1);
+        const uint32_t drawLength = drawn - hgt;
+        CkdSpan sp;
+        ckd_span_setup_drawn(sp, color, lastColor, length, drawLength, udiv24(65536u, length));
+        global_u32 *p = row + (W - drawn);
+        for (uint32_t j = 0; j < drawLength; ++j) {
+            p[j] = ckd_span_pixel(sp.acc);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sp.acc[c] += sp.step[c];
         }
     }
     const uint32_t sky = fog[0];
-    for (unsigned x = written; x < W; ++x) row[x] = sky;
+    for (unsigned x = W - (unsigned)top + lane; x < W; x += 64) row[x] = sky;
 }
 
 ckd_status upload(const void *host, size_t bytes, void **dev)
@@ -722,15 +773,13 @@ ckd_status ckd_tunnelscape_rows(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigne
     if (!ctx->tsHeight)
         return ckd::fail(CKD_ESTATE, "ckd_tunnelscape_rows: no maps (ckd_tunnelscape_create)");
     // tscape (code/tunnelscape.cpp:103-118) frame constants, host FP32
-    float mapStepX, fromXAdd, kMapViewLenScale;
+    float mapStepX, fromXAdd;
     int dX, dY, fpFromY;
     {
 #pragma clang fp contract(off)
         const float kGoldenRatio = 1.61803398875f;
         const float aspect = (float)H / (float)W;
         const float kOneOverAspect = 1.f / aspect;
-        // kMapViewLenScale is the reference's 720p constant (code/tunnelscape.cpp:31)
-        kMapViewLenScale = (720.f / 1280.f) * 0.5f;
         mapStepX = 2048.f / (float)(H - 1);
         const float speedMul = sqrtf(stepU * stepU + stepV * stepV) * speed;
         const float fromY = 1024.f + speedMul * time;
@@ -739,9 +788,8 @@ ckd_status ckd_tunnelscape_rows(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigne
         fpFromY = (int)(fromY * 256.f);
         fromXAdd = stepU * time * kGoldenRatio;
     }
-    k_tunnelscape<<<ckd_div_up(H, 64), 64, 0, ctx->stream>>>(dst, W, H, ctx->tsHeight, ctx->tsColor,
-                                                            ctx->tsFog, mapStepX, fromXAdd, fpFromY,
-                                                            dX, dY, kMapViewLenScale);
+    k_tunnelscape<<<H, 64, 0, ctx->stream>>>(dst, W, H, ctx->tsHeight, ctx->tsColor, ctx->tsFog, mapStepX,
+                                             fromXAdd, fpFromY, dX, dY);
     return ckd::check_launch("tunnelscape");
 }
 
