@@ -15,10 +15,10 @@
 //
 // In place (dst == src) the reference's subtract reads pixels it has
 // already overwritten, which makes every line a sequential recurrence with
-// u16 saturation; those kernels run one lane per line and channel and
-// replay it, on lines staged in LDS (k_blur07_lines) or with an LDS ring of
-// the recent outputs per lane, reading the image directly
-// (k_blur07_ring_*).
+// u16 saturation.  Small batches run it as scans of chunks of steps, a wave
+// per line (k_blur07_scan_*); large ones replay it with one lane per line and
+// channel, on lines staged in LDS (k_blur07_lines) or with an LDS ring of the
+// recent outputs per lane, reading the image directly (k_blur07_ring_*).
 #include "ckd_internal.h"
 #include "ckd_pixel.h"
 #include "ckd_b07.h"
@@ -632,6 +632,224 @@ __global__ __launch_bounds__(kRingBlock) void k_blur07_ring_one(B07Job job, int 
     b07_ring_block<K, false>(job, nLines, len, columns, ringLen, nullptr, ringBuf, divs);
 }
 
+// The in-place blur as a scan, for batches that leave the lane-per-line
+// kernels above short of waves (their time is one line's chain of steps, 44 to
+// 85 ns a step).  A step is
+//   acc = max(min(acc + a, 65535) - s, 0) = clamp(acc + (a - s), 0, 65535 - s)
+// with a from the pixel entering and s from the output made `median` steps
+// earlier.  Clamped additions are closed under composition: x -> clamp(x + d,
+// l, h) followed by (d2, l2, h2) is
+//   (d + d2, clamp(l + d2, l2, h2), clamp(h + d2, l2, h2)),
+// so the kSteps <= median steps of a chunk, whose s are all known, are a prefix
+// scan over lanes.  One wave per line, the line staged in LDS: lane (channel, t)
+// of four rows of 16 lanes takes step t of the chunk, and the scan runs inside
+// the rows on DPP shifts.  Lane 0 applies its step to the carried acc, which
+// makes it a constant (l = h = acc); a lane whose shift reaches past the row's
+// start is constant already, and clamping anything into [l, l] gives l, so the
+// zeros shifted in do no harm.
+// Step p adds pixel p (0 from len on), subtracts output p - span and makes
+// output p - edge: the reference's four phases (code/deprecated/boxblur.cpp:
+// 81-125) in one form, with zeros where a phase adds or subtracts nothing.
+// What bounds it: one wave's issue, about 45 instructions a chunk, and the LDS
+// latency between a chunk's outputs and the next one's reads.  One 1280x720
+// image, span 82: rows 74 -> 21 us, columns 71 -> 18 us.  Reading the
+// subtracted outputs a chunk ahead too, where the median allows it, was no
+// faster.
+constexpr int kScanLines = 4; // lines (waves) per block
+constexpr int kScanPad = 17;  // words past a line: the middle run's lookahead stays below 16
+
+// A chunk's scan: step (d, 0, h) in each lane, carry the acc before the chunk;
+// returns the lane's acc and moves carry on to lane kSteps - 1's.  One asm
+// block: a VALU result needs two instructions between it and the DPP that
+// reads it, which the order here gives (or an s_nop), and the medians are
+// clamps, lo <= hi, which the compiler cannot know.
+#define B07_SHR(N) " row_shr:" #N " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+// one level, (d, l, h) -> (D, L, h); T is scratch
+#define B07_LEVEL(N, d, l, D, L)                                      \
+    "v_add_u32_dpp %[" D "], %[" d "], %[" d "]" B07_SHR(N)           \
+    "v_add_u32_dpp %[" L "], %[" l "], %[" d "]" B07_SHR(N)           \
+    "v_add_u32_dpp %[t], %[h], %[" d "]" B07_SHR(N)                   \
+    "v_med3_i32 %[" L "], %[" L "], %[" l "], %[h]\n"                 \
+    "v_med3_i32 %[h], %[t], %[" l "], %[h]\n"
+// the last level: only l is wanted, then its lane B to the whole row
+#define B07_LAST(N, d, l, L, B)                                       \
+    "s_nop 0\n"                                                       \
+    "v_add_u32_dpp %[" L "], %[" l "], %[" d "]" B07_SHR(N)           \
+    "v_med3_i32 %[" L "], %[" L "], %[" l "], %[h]\n"                 \
+    "s_nop 1\n"                                                       \
+    "v_mov_b32_dpp %[c], %[" L "] row_newbcast:" #B " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+#define B07_FIRST                                                     \
+    "v_add_u32 %[t], %[c], %[d]\n"                                    \
+    "v_med3_i32 %[t], %[t], 0, %[h]\n"                                \
+    "v_cndmask_b32 %[l], 0, %[t], %[m]\n"                             \
+    "v_cndmask_b32 %[h], %[h], %[t], %[m]\n"
+#define B07_OPERANDS                                                                                     \
+    : [d] "+v"(d), [h] "+v"(h), [c] "+v"(carry), [l] "=&v"(l), [L] "=&v"(L), [D] "=&v"(D), [t] "=&v"(t) \
+    : [m] "s"(0x0001000100010001ull)
+#define B07_SCAN16(B)                                                                                  \
+    asm(B07_FIRST B07_LEVEL(1, "d", "l", "D", "L") B07_LEVEL(2, "D", "L", "d", "l")                      \
+        B07_LEVEL(4, "d", "l", "D", "L") B07_LAST(8, "D", "L", "l", B) B07_OPERANDS)
+#define B07_SCAN8(B)                                                                                   \
+    asm(B07_FIRST B07_LEVEL(1, "d", "l", "D", "L") B07_LEVEL(2, "D", "L", "d", "l")                      \
+        B07_LAST(4, "d", "l", "L", B) B07_OPERANDS)
+template <int kSteps> CKD_DEV int b07_scan(int d, int h, int &carry)
+{
+    static_assert(kSteps == 16 || kSteps == 12 || kSteps == 10 || kSteps == 8 || kSteps == 6 || kSteps == 4,
+                  "steps per chunk");
+    int l, L, D, t;
+    if constexpr (kSteps == 16) B07_SCAN16(15);
+    if constexpr (kSteps == 12) B07_SCAN16(11);
+    if constexpr (kSteps == 10) B07_SCAN16(9);
+    if constexpr (kSteps == 8) B07_SCAN8(7);
+    if constexpr (kSteps == 6) B07_SCAN8(5);
+    if constexpr (kSteps == 4)
+        asm(B07_FIRST B07_LEVEL(1, "d", "l", "D", "L") B07_LAST(2, "D", "L", "l", 3) B07_OPERANDS);
+    return kSteps == 8 || kSteps == 6 ? L : l;
+}
+#undef B07_SCAN16
+#undef B07_SCAN8
+#undef B07_SHR
+#undef B07_LEVEL
+#undef B07_LAST
+#undef B07_FIRST
+#undef B07_OPERANDS
+
+// One channel of one line: px is its byte in the line's pixel 0 (LDS), t the
+// lane's step in a chunk.  split: stop before the step that adds the line's
+// last pixel and save the state (b07_lds_line's kSplit).
+template <int kSteps, bool kEven>
+CKD_DEV void b07_scan_line(uint8_t *px, int len, const B07Params &p, const uint16_t *divs, int t, bool split,
+                           uint32_t *state)
+{
+    const int e = (int)p.edgeSpan, m = (int)p.median, em = e + m;
+    const int fullDiv = (int)p.fullDiv;
+    const int nSteps = split ? len - 1 : len + e;
+    int carry = 0;
+    // the scan of a chunk's steps from its inputs (x1, the pixel before it
+    // x0) and outputs made a span earlier (y1, y0); returns the lane's acc
+    auto scan = [&](int x1, int x0, int y1, int y0) {
+        const int a = kEven ? x1 - (x1 >> 1) + (x0 >> 1) : x1, s = kEven ? y1 - (y1 >> 1) + (y0 >> 1) : y1;
+        return b07_scan<kSteps>(a - s, 65535 - s, carry);
+    };
+    // Div + packus_epi16 (code/deprecated/boxblur.cpp:39-42)
+    auto quotient = [](int acc, int div) {
+        const int q = (int)ckd_mul_u24_v((uint32_t)acc, (uint32_t)div) >> 16;
+        return (uint8_t)min(max(q, 0), 255);
+    };
+    // a chunk anywhere
+    auto edge_chunk = [&](int p0) {
+        const int pos = p0 + t, out = pos - e, back = pos - em;
+        const int x1 = pos < len ? (int)px[4 * min(pos, len - 1)] : 0;
+        const int x0 = pos > 0 && pos <= len ? (int)px[4 * max(min(pos, len) - 1, 0)] : 0;
+        const int y1 = back >= 0 && t < kSteps ? (int)px[4 * max(back, 0)] : 0;
+        const int y0 = back > 0 && t < kSteps ? (int)px[4 * max(back - 1, 0)] : 0;
+        const int acc = scan(x1, x0, y1, y0);
+        int div = fullDiv;
+        if (out < m) div = divs[max(out, 0)];
+        else if (out >= len - e) div = divs[max(len - 1 - out, 0)];
+        if (t < kSteps && out >= 0 && pos < nSteps) px[4 * out] = quotient(acc, div);
+        if (split && pos == nSteps - 1 && t < kSteps) {
+            state[0] = (uint32_t)acc;
+            state[1] = kEven ? (uint32_t)(x1 >> 1) : 0u;
+            state[2] = kEven ? (uint32_t)(y1 >> 1) : 0u;
+        }
+    };
+    int p0 = 0;
+    for (; p0 <= em && p0 < nSteps; p0 += kSteps) edge_chunk(p0);
+    // whole chunks inside the middle run: back > 0, pos < len - 1 and pos <
+    // nSteps, full divisor; the next chunk's pixels are read ahead
+    const int last = len - 1 - 16;
+    if (p0 <= last) {
+        const uint8_t *in = px + 4 * (p0 + t), *from = in - 4 * em;
+        uint8_t *to = px + 4 * (p0 + t - e);
+        int x1 = in[0], x0 = kEven ? (int)in[-4] : 0;
+        for (; p0 <= last; p0 += kSteps) {
+            const int y1 = from[0], y0 = kEven ? (int)from[-4] : 0;
+            in += 4 * kSteps;
+            from += 4 * kSteps;
+            const int n1 = in[0], n0 = kEven ? (int)in[-4] : 0;
+            const int acc = scan(x1, x0, y1, y0);
+            if (kSteps == 16 || t < kSteps) *to = quotient(acc, fullDiv);
+            to += 4 * kSteps;
+            x1 = n1;
+            x0 = n0;
+        }
+    }
+    for (; p0 < nSteps; p0 += kSteps) edge_chunk(p0);
+}
+
+template <int kSteps>
+CKD_DEV void b07_scan_block(const B07Job &J, int nLines, int len, int columns, unsigned block, uint32_t *states,
+                            uint32_t *lineBuf)
+{
+    __shared__ uint16_t divs[256];
+    const int tid = threadIdx.x, nThreads = blockDim.x, nl = nThreads >> 6;
+    const int line0 = (int)block * nl, lines = min(nl, nLines - line0);
+    const int stride = len + kScanPad;
+    for (int i = tid; i < 256; i += nThreads) divs[i] = J.p.edgeDivs[i];
+    global_px32 *img = (global_px32 *)J.img;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // rows: each wave moves its own line; columns: a row of nl (a power of two)
+    // pixels after the other.  Eight pixels per thread in flight.
+    const int nlLog2 = __builtin_ctz((unsigned)nl);
+    const int l = columns ? tid & (nl - 1) : wave, x0 = columns ? tid >> nlLog2 : lane, dx = 64;
+    const uint32_t at = columns ? (uint32_t)(line0 + l) : (uint32_t)(line0 + l) * (uint32_t)len;
+    const uint32_t pstep = columns ? (uint32_t)nLines : 1u;
+    uint32_t *mine = lineBuf + l * stride;
+    if (l < lines) {
+        for (int x = x0; x < len; x += 8 * dx) {
+            uint32_t v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = img[at + (uint32_t)min(x + k * dx, len - 1) * pstep];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (x + k * dx < len) mine[x + k * dx] = v[k];
+        }
+    }
+    __syncthreads();
+    const int ch = lane >> 4, t = lane & 15;
+    if (wave < lines) {
+        uint8_t *px = reinterpret_cast<uint8_t *>(lineBuf + wave * stride) + ch;
+        uint32_t *st = states ? states + ((size_t)(line0 + wave) * 4 + ch) * 3 : nullptr;
+        if (J.p.subEdges) b07_scan_line<kSteps, true>(px, len, J.p, divs, t, states != nullptr, st);
+        else b07_scan_line<kSteps, false>(px, len, J.p, divs, t, states != nullptr, st);
+    }
+    __syncthreads();
+    if (l < lines)
+#pragma unroll 8
+        for (int x = x0; x < len; x += dx) img[at + (uint32_t)x * pstep] = mine[x];
+}
+
+// consecutive blocks on one XCD: columns of one cache line then meet in its L2
+CKD_DEV unsigned scan_block_of(unsigned blocks)
+{
+    return (blockIdx.x & 7) * ((blocks + 7) / 8) + (blockIdx.x >> 3);
+}
+
+// blockIdx.y picks the job
+template <int kSteps>
+__global__ __launch_bounds__(kScanLines * 64) void k_blur07_scan_jobs(const B07Job *__restrict__ jobs, int nLines,
+                                                                     int len, int columns, unsigned blocks,
+                                                                     uint32_t *__restrict__ states)
+{
+    extern __shared__ uint32_t lineBuf[];
+    const unsigned b = scan_block_of(blocks);
+    if (b >= blocks) return;
+    b07_scan_block<kSteps>(jobs[blockIdx.y], nLines, len, columns, b,
+                           states ? states + (size_t)blockIdx.y * nLines * 12 : nullptr, lineBuf);
+}
+
+// one image, its job passed by value
+template <int kSteps>
+__global__ __launch_bounds__(kScanLines * 64) void k_blur07_scan_one(B07Job job, int nLines, int len, int columns,
+                                                                    unsigned blocks)
+{
+    extern __shared__ uint32_t lineBuf[];
+    const unsigned b = scan_block_of(blocks);
+    if (b >= blocks) return;
+    b07_scan_block<kSteps>(job, nLines, len, columns, b, nullptr, lineBuf);
+}
+
 // the chain of a batch of render targets whose last column carries from one
 // image to the next (the ball's frames with beams): one lane per line and
 // channel walks the images in order.  mode 0: the image's last column is
@@ -757,10 +975,57 @@ int ring_len(unsigned mHi)
 size_t ring_lds(int ringLen) { return (size_t)kRingBlock * (size_t)(ringLen + 4); }
 int ring_k(unsigned mLo) { return mLo >= 8 ? 8 : mLo >= 4 ? 4 : mLo >= 2 ? 2 : 1; }
 
+// The scan kernel's steps per chunk: the most of 16, 12, 10, 8, 6, 4 that the
+// smallest median of the batch allows (0: none); its lines per block (their LDS
+// within 64 KiB) and its grid.  One wave takes a line, so its time grows with
+// the lines per SIMD and with the chunks of a line, where the kernels above
+// take one line's time until they have filled the chip: it is taken up to (steps
+// - 2) * 5 / 4 lines per SIMD.  Measured at 1280x720, rows and columns, us,
+// scan against the better of the others: span 82 (16 steps) 1 frame 21 and 18
+// against 74 and 71, 8 frames 48 and 50 against 75 and 88, 16 frames 85 and 83
+// against 151 and 90, 48 frames 218 and 223 against 206 and 146; span 22 (10
+// steps) 8 frames 71 and 70 against 75 and 86, 16 frames 131 and 122 against
+// 148 and 88; span 10 (4 steps) 8 frames 113 and 104 against 80 and 86.
+struct ScanShape {
+    int steps = 0, lines = 0;
+    unsigned blocks = 0;
+    size_t lds = 0;
+    dim3 grid(unsigned n) const { return dim3((blocks + 7) / 8 * 8, n); }
+};
+ScanShape scan_shape(const ckd_ctx *ctx, unsigned mLo, int nLines, int len, unsigned n)
+{
+    ScanShape S;
+    const size_t line = (size_t)(len + kScanPad) * 4;
+    if (mLo < 4 || line > 65536) return S;
+    const int steps = mLo >= 16 ? 16 : mLo >= 12 ? 12 : mLo >= 10 ? 10 : mLo >= 8 ? 8 : mLo >= 6 ? 6 : 4;
+    if ((size_t)nLines * n * 4 > (size_t)(steps - 2) * 5 * 4 * (size_t)ctx->cuCount) return S;
+    S.steps = steps;
+    S.lines = kScanLines;
+    while ((size_t)S.lines * line > 65536) S.lines >>= 1;
+    S.lds = (size_t)S.lines * line;
+    S.blocks = ckd_div_up((size_t)nLines, (size_t)S.lines);
+    return S;
+}
+
 ckd_status launch_inplace(ckd_ctx *ctx, uint32_t *img, int nLines, int len, size_t lineStride,
                           size_t pixStride, const B07Params &p, const char *what)
 {
     const int nl = lines_per_block(len);
+    if (const ScanShape S = scan_shape(ctx, p.median, nLines, len, 1); S.steps) {
+        B07Job job;
+        job.img = img;
+        job.p = p;
+        const int columns = pixStride != 1 ? 1 : 0, threads = S.lines * 64;
+        switch (S.steps) {
+        case 16: k_blur07_scan_one<16><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        case 12: k_blur07_scan_one<12><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        case 10: k_blur07_scan_one<10><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        case 8: k_blur07_scan_one<8><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        case 6: k_blur07_scan_one<6><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        default: k_blur07_scan_one<4><<<S.grid(1), threads, S.lds, ctx->stream>>>(job, nLines, len, columns, S.blocks); break;
+        }
+        return ckd::check_launch(what);
+    }
     if (pixStride != 1 || nl == 0) {
         // columns (the ring kernel reads them coalesced across the wave,
         // where staging strided columns in LDS is slow), or lines longer
@@ -881,6 +1146,19 @@ ckd_status blur07_inplace_jobs(ckd_ctx *ctx, const B07Job *hostJobs, const B07Jo
         ring = columns || blocks > perCU * (size_t)ctx->cuCount;
     }
     const char *what = columns ? "blur07_v (in place, batch)" : "blur07_h (in place, batch)";
+    const ScanShape S = ctx->tuning.blurKernel == 0 ? scan_shape(ctx, mLo, (int)nLines, (int)len, n) : ScanShape();
+    if (S.steps) {
+        const int cols = columns ? 1 : 0, threads = S.lines * 64;
+        switch (S.steps) {
+        case 16: k_blur07_scan_jobs<16><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        case 12: k_blur07_scan_jobs<12><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        case 10: k_blur07_scan_jobs<10><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        case 8: k_blur07_scan_jobs<8><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        case 6: k_blur07_scan_jobs<6><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        default: k_blur07_scan_jobs<4><<<S.grid(n), threads, S.lds, ctx->stream>>>(devJobs, (int)nLines, (int)len, cols, S.blocks, splitStates); break;
+        }
+        return check_launch(what);
+    }
     if (ring) {
         const int ringLen = ring_len(mHi);
         const int K = ring_k(mLo);
