@@ -6,7 +6,11 @@
 
 #include <cstdint>
 
-// SDF request: 32x32-pixel chunks are the units of the persistent queue
+// the SDF chunk queues' counters: kSdfQueues words, kSdfQueueStride words apart
+// (a memory channel each), at the start of the staged tables
+constexpr uint32_t kSdfQueues = 8, kSdfQueueStride = 64;
+
+// SDF request: square pixel chunks are the units of the persistent queue
 struct SdfJob {
     uint32_t *dst;
     uint32_t W, H;

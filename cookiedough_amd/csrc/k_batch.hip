@@ -3,7 +3,7 @@
 //
 // The host sorts the requests into three job tables (SDF, voxel, tunnel)
 // and stages them in one device buffer together with the SDF chunk-queue
-// counter.  One persistent SDF kernel runs on the context stream; the voxel
+// counters.  One persistent SDF kernel runs on the context stream; the voxel
 // kernel (every voxel column of every request) and the two fused tunnel
 // kernels run beside it on the auxiliary stream.  The same launch sequence
 // is replayed eagerly (ckd_render_batch), timed over candidate launch
@@ -16,10 +16,11 @@
 #include <vector>
 
 namespace ckd {
-ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t totalChunks,
+ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t totalChunks, uint32_t side,
                                  const SdfJob *jobs, int nJobs, const ckd_sdf_scene &sc,
                                  int shading, unsigned long long *stepCount, bool helper,
                                  bool alone);
+uint32_t sdf_chunk_side(int tuned, size_t pixels, int nSpheres);
 void voxel_job_geometry(VoxJob &J, unsigned W, unsigned H, const ckd_landscape_cam &c);
 unsigned voxel_block_cols(size_t columns);
 ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, uint32_t totalBlocks,
@@ -50,10 +51,11 @@ struct ckd_graph {
     hipGraphExec_t exec = nullptr;
     bool hasSdf = false;
     // what ckd_graph_update must keep: the launch shapes the tables were
-    // laid out with, the scratch image, the requests' shapes
+    // laid out with, the scratch image, the scene's size, the requests' shapes
     ckd_tuning tuning{};
     uint32_t *tmp = nullptr;
     size_t tmpPixels = 0;
+    int nSpheres = 0;
     std::vector<ReqShape> shapes;
     // window rows of the captured vertical-blur ring (0: no ring): the
     // largest radius a replay can take
@@ -65,18 +67,19 @@ namespace {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// host image of the staged tables: [queue counter][SDF][voxel][tunnel]
+// host image of the staged tables: [queue counters][SDF][voxel][tunnel]
 struct Plan {
     std::vector<unsigned char> host;
-    size_t oSdf = 256, oVox = 0, oTun = 0;
+    size_t oSdf = kSdfQueues * kSdfQueueStride * sizeof(uint32_t), oVox = 0, oTun = 0;
     int nSdf = 0, nVox = 0, nTun = 0;
     uint32_t chunks = 0, voxBlocks = 0, tunRows = 0, tunV = 0;
+    uint32_t sdfSide = 0; // side of the SDF chunks
     unsigned voxCols = 0; // columns per voxel block
     unsigned tunMaxW = 0;
     unsigned tunMaxE = 0;
 };
 
-__global__ void k_reset_counter(uint32_t *c) { *c = 0u; }
+__global__ void k_reset_counters(uint32_t *c) { c[kSdfQueueStride * threadIdx.x] = 0u; }
 
 ckd_status validate(const char *fn, const ckd_request *requests, unsigned n,
                     const ckd_sdf_scene *scene, int shading, const uint32_t *tex, unsigned texLog2,
@@ -123,15 +126,17 @@ ckd_status validate(const char *fn, const ckd_request *requests, unsigned n,
 }
 
 void make_plan(const ckd_tuning &T, const ckd_request *requests, unsigned n, uint32_t *tmp,
-               Plan &P)
+               int nSpheres, Plan &P)
 {
     std::vector<SdfJob> sdf;
     std::vector<VoxJob> vox;
     std::vector<TunJob> tun;
-    const uint32_t chunk = (uint32_t)T.sdfChunk;
-    size_t off = 0, voxColumns = 0;
-    for (unsigned i = 0; i < n; ++i)
+    size_t off = 0, voxColumns = 0, sdfPixels = 0;
+    for (unsigned i = 0; i < n; ++i) {
         if (requests[i].effect == CKD_FX_VOXEL) voxColumns += requests[i].W;
+        if (requests[i].effect == CKD_FX_SDF) sdfPixels += (size_t)requests[i].W * requests[i].H;
+    }
+    const uint32_t chunk = P.sdfSide = ckd::sdf_chunk_side(T.sdfChunk, sdfPixels, nSpheres);
     P.voxCols = ckd::voxel_block_cols(voxColumns);
     for (unsigned i = 0; i < n; ++i) {
         const ckd_request &r = requests[i];
@@ -189,7 +194,7 @@ ckd_status launch_plan(ckd_ctx *ctx, const Plan &P, unsigned char *dev, const ck
         CKD_HIP(hipStreamWaitEvent(ctx->aux, ctx->forkEv, 0));
     }
     if (P.nSdf > 0) {
-        s = ckd::launch_sdf_persistent(ctx, reinterpret_cast<uint32_t *>(dev), P.chunks,
+        s = ckd::launch_sdf_persistent(ctx, reinterpret_cast<uint32_t *>(dev), P.chunks, P.sdfSide,
                                        reinterpret_cast<const SdfJob *>(dev + P.oSdf), P.nSdf,
                                        *scene, shading, stepCount, false, !fork);
         if (s != CKD_OK) return s;
@@ -224,7 +229,7 @@ ckd_status launch_plan(ckd_ctx *ctx, const Plan &P, unsigned char *dev, const ck
         if (split) CKD_HIP(hipStreamWaitEvent(ctx->aux, ctx->tunEv, 0));
         if (fork) {
             // the voxel / tunnel work is done: its CUs join the SDF march
-            s = ckd::launch_sdf_persistent(ctx, reinterpret_cast<uint32_t *>(dev), P.chunks,
+            s = ckd::launch_sdf_persistent(ctx, reinterpret_cast<uint32_t *>(dev), P.chunks, P.sdfSide,
                                            reinterpret_cast<const SdfJob *>(dev + P.oSdf), P.nSdf,
                                            *scene, shading, stepCount, true, false);
             if (s != CKD_OK) return s;
@@ -242,7 +247,7 @@ ckd_status run_eager(ckd_ctx *ctx, const ckd_request *requests, unsigned n,
                      unsigned texLog2, uint32_t *tmp, unsigned long long *stepCount)
 {
     Plan P;
-    make_plan(ctx->tuning, requests, n, tmp, P);
+    make_plan(ctx->tuning, requests, n, tmp, scene ? scene->nSpheres : 0, P);
     void *dev = nullptr;
     ckd_status s = ckd::stage(ctx, P.host.data(), P.host.size(), &dev);
     if (s != CKD_OK) return s;
@@ -391,12 +396,13 @@ ckd_status ckd_batch_graph_create(ckd_ctx *ctx, const ckd_request *requests, uns
     CKD_REQUIRE(n > 0, "ckd_batch_graph_create: empty batch");
     CKD_REQUIRE_CTX(ctx);
     Plan P;
-    make_plan(ctx->tuning, requests, n, tmp, P);
+    make_plan(ctx->tuning, requests, n, tmp, scene ? scene->nSpheres : 0, P);
     ckd_graph *g = new ckd_graph();
     g->ctx = ctx;
     g->tableBytes = P.host.size();
     g->tuning = ctx->tuning;
     g->tmp = tmp;
+    g->nSpheres = scene ? scene->nSpheres : 0;
     g->tmpPixels = tmpPixels;
     g->tunRingRows = P.nTun ? ckd::tunnel_ring_rows(P.tunMaxE) : 0;
     for (unsigned i = 0; i < n; ++i)
@@ -429,8 +435,8 @@ ckd_status ckd_batch_graph_create(ckd_ctx *ctx, const ckd_request *requests, uns
     if (e == hipSuccess) {
         ckd::StreamSwap swap(ctx, cap);
         unsigned char *dev = static_cast<unsigned char *>(g->tables);
-        // the queue counter is reset by a kernel node on every replay
-        k_reset_counter<<<1, 1, 0, cap>>>(reinterpret_cast<uint32_t *>(dev));
+        // the queue counters are reset by a kernel node on every replay
+        k_reset_counters<<<1, kSdfQueues, 0, cap>>>(reinterpret_cast<uint32_t *>(dev));
         s = launch_plan(ctx, P, dev, scene, shading, tex, g->quads, texLog2, stepCount);
         const hipError_t e2 = hipStreamEndCapture(cap, &g->graph);
         if (s == CKD_OK && e2 != hipSuccess)
@@ -476,7 +482,7 @@ ckd_status ckd_graph_update(ckd_graph *g, const ckd_request *requests, unsigned 
         }
     }
     Plan P;
-    make_plan(g->tuning, requests, n, g->tmp, P);
+    make_plan(g->tuning, requests, n, g->tmp, g->nSpheres, P);
     if (P.host.size() != g->tableBytes)
         return ckd::fail(CKD_EINVAL, "ckd_graph_update: the requests' tables do not fit the graph");
     if (g->tunRingRows && 2 * P.tunMaxE + 1 > g->tunRingRows)

@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 
 namespace {
@@ -206,8 +207,11 @@ __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigne
 
 // ---- persistent batched tracer ------------------------------------------
 //
-// One launch renders every SDF request of a batch.  Each wave pulls 32x32
-// pixel chunks from a global queue (one atomic per chunk).  Inside a chunk
+// One launch renders every SDF request of a batch.  Each wave pulls square
+// pixel chunks (sdf_chunk_side) from global queues (one atomic per chunk).
+// At its start it finds the spheres that can be the nearest surface anywhere
+// on the chunk's rays (chunk_spheres); the march evaluates only those.  Inside
+// a chunk
 // the wave keeps its 64 lanes busy: lanes whose ray has finished are
 // refilled with the chunk's next pixels (ballot + mbcnt ranks), so a
 // long-marching ray no longer holds 63 idle lanes.  Finished rays are
@@ -270,6 +274,9 @@ CKD_DEV uint32_t opaque_zero()
     asm volatile("s_mov_b32 %0, 0" : "=s"(z));
     return z;
 }
+
+// lane k's value, in a scalar register
+CKD_DEV float lane_f(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }
 
 // a wave-uniform float kept in a scalar register
 CKD_DEV float uniform_f(float v)
@@ -362,9 +369,88 @@ CKD_DEV uint32_t shade_hit(const ckd_sdf_scene &sc, const float *cam, float dx, 
     return shade_lit<kHalf>(sc, m, nx, ny, nz, id);
 }
 
+// far above the rounding of distances in a scene of that scale, |b|^2 = bb from
+// the camera to the bounding sphere's centre
+CKD_DEV float cull_margin(float bb, float R) { return fmaf(1e-4f, fsqrt(bb) + R, 1e-3f); }
+
+// The stretch (tNear, tFar) of a ray outside which no sphere can be nearer than
+// the ground.  Every sphere lies inside the bounding sphere (centre C, radius
+// R; b = o - C), so each one's distance is at least |p - C| - R; where that is
+// at least the ground's distance g plus a margin the ground is the minimum.
+// With p = o + t d and g = og + t dy that is
+//   (t + m)^2 + |b|^2 - m^2 >= (a + c t)^2,  m = d.b,
+//   a = 1.001 og + R + margin,  c = 1.001 dy,
+// (or a + c t < 0, where it holds anyway): true outside the roots of
+//   (1 - c^2) t^2 + 2 (m - a c) t + |b|^2 - a^2.
+// The margin, 1e-3 + 1e-4 (|b| + R) + 1e-3 g, is far above the rounding of the
+// roots and of either side (about 1e-6 of the scene's scale), also where the
+// discriminant nearly vanishes: a wrong sign there moves the test by less than
+// the margin.  g < 0 beyond that is met only at the first step of a camera
+// below the ground: such rays, and near-vertical ones (1 - c^2 small), get the
+// whole line.  Against evaluating the bound at every step this takes 4 VALU of
+// a step's 14 (64 frames of 1280x720: 1459 -> 1390 us).
+// spread: bound of |d' - d| over the rays d' the stretch has to hold for (their
+// points at t lie within t * spread of the ray's, which moves either side of
+// the test by that much).
+CKD_DEV void near_interval(float bx, float by, float bz, float R, float og, float dx, float dy, float dz,
+                           float spread, float &tNear, float &tFar)
+{
+    const float bb = bx * bx + by * by + bz * bz;
+    const float m = dx * bx + dy * by + dz * bz;
+    const float a = fmaf(1.001f, og, R + cull_margin(bb, R)), c = fmaf(1.001f, dy, 2.002f * spread);
+    const float A = fmaf(-c, c, 1.f), B = fmaf(-a, c, m);
+    const float disc = fmaf(B, B, -A * (bb - a * a));
+    const float s = fsqrt(fmaxf(disc, 0.f)), inv = __builtin_amdgcn_rcpf(A);
+    tNear = (-B - s) * inv;
+    tFar = (-B + s) * inv;
+    if (disc < 0.f || tFar < 0.f) tNear = INFINITY;
+    if (!(A > 0.01f) || !(og > 0.f) || !(disc == disc)) {
+        tNear = -INFINITY;
+        tFar = INFINITY;
+    }
+}
+
 // lanes that must be idle before a wave refills them (checked every
 // kStepsPerRefill march steps)
 constexpr int kRefillMinIdle = 32;
+
+// The spheres that can be the nearest surface to some point of a chunk's rays,
+// as a bit mask.  The chunk's rays stay within t * spread of its central ray
+// (d; spread bounds |d' - d| over the chunk).  The stretch of it that can be
+// near any sphere is cut into 64 pieces, one per lane: every point of a ray in
+// the piece lies within rho of the piece's middle q, and a distance changes by
+// no more than the way moved.  The nearest surface at such a point is at most
+// m + rho away, m the scene's distance at q, so a sphere whose distance at q
+// exceeds m + 2 rho (and the rounding margin) is not the nearest anywhere in
+// the piece.  One that no piece needs can be left out of the chunk's minimum,
+// which stays the same to the bit.  64 frames of 1280x720 with 8 spheres: 1213
+// -> 1101 us; 24 of 2560x1440 with 32: 5273 -> 2962 us.
+CKD_DEV uint32_t chunk_spheres(const ckd_sdf_scene &sc, const float *cam, const f4 &bound, float bx, float by, float bz,
+                               float dx, float dy, float dz, float spread, uint32_t lane, uint32_t all)
+{
+    const float og = cam[1] - sc.groundY, bb = bx * bx + by * by + bz * bz;
+    float t0, t1;
+    near_interval(bx, by, bz, bound.w, og, dx, dy, dz, spread, t0, t1);
+    t0 = fmaxf(t0, 0.f);
+    t1 = fminf(t1, sc.tMax);
+    if (__builtin_amdgcn_readfirstlane(t0 >= t1)) return 0;
+    if (__builtin_amdgcn_readfirstlane(!(t1 < 1e6f))) return all;
+    const float h = (t1 - t0) * (1.f / 64.f), t = fmaf((float)lane + 0.5f, h, t0);
+    const float rho = fmaf(t + h, spread, 0.5f * h);
+    const float qx = fmaf(t, dx, cam[0]), qy = fmaf(t, dy, cam[1]), qz = fmaf(t, dz, cam[2]);
+    auto distance = [&](int i) {
+        const float ex = qx - sc.sphere[i][0], ey = qy - sc.sphere[i][1], ez = qz - sc.sphere[i][2];
+        return fsqrt(ex * ex + ey * ey + ez * ez) - sc.sphere[i][3];
+    };
+    float m = qy - sc.groundY;
+#pragma unroll 4
+    for (int i = 0; i < sc.nSpheres; ++i) m = fminf(m, distance(i));
+    const float reach = fmaf(2.002f, rho, m) + cull_margin(bb, bound.w) + 1e-3f * fabsf(m);
+    uint32_t keep = 0;
+#pragma unroll 1
+    for (int i = 0; i < sc.nSpheres; ++i) keep |= __ballot(!(distance(i) > reach)) ? 1u << i : 0u;
+    return keep;
+}
 
 template <bool kHalf, int kMaxSph, int kStepsPerRefill>
 __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uint32_t *__restrict__ queueCounter,
@@ -372,7 +458,7 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
                                                         const SdfJob *__restrict__ jobs, int nJobs,
                                                         const ckd_sdf_scene sc,
                                                         unsigned long long *__restrict__ stepCount,
-                                                        uint32_t kChunkSide, f4 bound,
+                                                        uint32_t kChunkSide, uint32_t fixedChunks, uint32_t nQueues, bool own, f4 bound,
                                                         unsigned long long *__restrict__ work)
 {
     __shared__ ShadeEntry queue[kWavesPerBlock][kQueueCap];
@@ -381,17 +467,21 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
     __shared__ f4 sphR[kWavesPerBlock][kMaxSph / 4]; // {r_4k .. r_4k+3}
     // o - c_i of the chunk's camera, read when a lane starts a ray
     __shared__ f4 sphOC[kWavesPerBlock][kMaxSph];
+    __shared__ uint32_t drained; // a wave of the block found the queue empty
+    if (threadIdx.x == 0) drained = 0;
+    __syncthreads();
     const uint32_t lane = lane_id();
-    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     ShadeEntry *q = queue[wave];
     int qn = 0; // entries waiting in this wave's queue (uniform)
 
     // chunk state (uniform)
     int job = -1;
-    uint32_t next = 0, end = 0, cx0 = 0, cy0 = 0, cw = 1, cwM = 1u << 20;
+    uint32_t next = 0, end = 0, cx0 = 0, cy0 = 0, tilesX = 1, tilesM = 1u << 20;
     float invH = 1.f;
     float cam[12];
     uint32_t W = 0, H = 0;
+    int sphGroups = 0; // the chunk's spheres (chunk_spheres), in groups of four
 
     // ray state (per lane)
     bool active = false;
@@ -399,11 +489,22 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
     // The ray's last march step evaluated the field at tHit and found d; its
     // distance total is t = tHit + d, which is how the step formed it, so t
     // is recomputed from the two instead of kept.  A new ray has tHit = -1
-    // and d = 1, so that t = 0.
-    float d = 1.f, tHit = -1.f, dx = 0.f, dy = 0.f, dz = 0.f;
+    // and d = 1, so that t = 0; a lane without a ray has tHit = inf, so that t
+    // = inf ends every march.
+    float d = 1.f, tHit = INFINITY, dx = 0.f, dy = 0.f, dz = 0.f;
     int steps = 0;
-    float M[kMaxSph], E2[kMaxSph]; // d.(o-c_i) and |w_i|^2 of the lane's ray
-    float Mb = 0.f, E2b = 0.f;     // the same for the centre of the spheres' bounding sphere
+    // d.(o-c_i) and |w_i|^2 of the lane's ray for the chunk's first spheres; the
+    // few chunks with more compute theirs where they need them
+    constexpr int kRegGroups = kMaxSph / 4 < 4 ? kMaxSph / 4 : 4;
+    float M[4 * kRegGroups], E2[4 * kRegGroups];
+    auto about_ray = [&](const f4 &oc, float &m, float &e2) {
+        m = dx * oc.x + dy * oc.y + dz * oc.z;
+        const float wx = fmaf(-m, dx, oc.x);
+        const float wy = fmaf(-m, dy, oc.y);
+        const float wz = fmaf(-m, dz, oc.z);
+        e2 = wx * wx + wy * wy + wz * wz;
+    };
+    float tNear = INFINITY, tFar = 0.f; // the ray needs the spheres for t between them only
     float bx = 0.f, by = 0.f, bz = 0.f; // o - C of the chunk's camera (uniform)
     unsigned long long mySteps = 0;
     // lane march steps of the wave that evaluated the spheres (uniform), and
@@ -420,32 +521,29 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
         if (idle && next < end && __popcll(idle) >= kRefillMinIdle) {
             const uint32_t rank = __popcll(idle & ((1ull << lane) - 1));
             if (!active) {
-                const uint32_t k = next + rank;
-                if (k < end) {
-                    // k / cw as (k * ceil(2^20 / cw)) >> 20, exact for k
-                    // < 4096 and cw <= 64
-                    const uint32_t row = __umul24(k, cwM) >> 20;
-                    const uint32_t x = cx0 + k - __umul24(row, cw), y = cy0 + row;
+                // the chunk's 8x8 tiles one after the other (rays of a tile
+                // march alike), row by row; tile / tilesX as (tile * ceil(2^20
+                // / tilesX)) >> 20, exact for tile < 4096 and tilesX <= 64
+                const uint32_t k = next + rank, tile = k >> 6;
+                const uint32_t ty = __umul24(tile, tilesM) >> 20;
+                const uint32_t x = cx0 + 8 * (tile - __umul24(ty, tilesX)) + (k & 7), y = cy0 + 8 * ty + ((k >> 3) & 7);
+                if (k < end && x < W && y < H) {
                     xy = x | (y << 16);
                     ray_dir(cam, W, H, invH, x, y, dx, dy, dz);
-                    const uint32_t z = opaque_zero();
+                    near_interval(bx, by, bz, bound.w, cam[1] - sc.groundY, dx, dy, dz, 0.f, tNear, tFar);
+                    if (__any(tNear < tFar)) {
+                        const uint32_t z = opaque_zero();
 #pragma unroll
-                    for (int i = 0; i < kMaxSph; ++i) {
-                        const f4 oc = sphOC[wave][i + z];
-                        const float m = dx * oc.x + dy * oc.y + dz * oc.z;
-                        const float wx = fmaf(-m, dx, oc.x);
-                        const float wy = fmaf(-m, dy, oc.y);
-                        const float wz = fmaf(-m, dz, oc.z);
-                        M[i] = m;
-                        E2[i] = wx * wx + wy * wy + wz * wz;
-                    }
-                    {
-                        const float m = dx * bx + dy * by + dz * bz;
-                        const float wx = fmaf(-m, dx, bx);
-                        const float wy = fmaf(-m, dy, by);
-                        const float wz = fmaf(-m, dz, bz);
-                        Mb = m;
-                        E2b = wx * wx + wy * wy + wz * wz;
+                        for (int g = 0; g < kRegGroups; ++g) {
+                            if (g >= sphGroups) break;
+#pragma unroll
+                            for (int i = 4 * g; i < 4 * g + 4; ++i) about_ray(sphOC[wave][i + z], M[i], E2[i]);
+                        }
+                    } else {
+                        // no ray of this refill needs a sphere: where the rest
+                        // of the wave makes them run the loop, none is near
+#pragma unroll
+                        for (int i = 0; i < 4 * kRegGroups; ++i) E2[i] = 1e30f;
                     }
                     d = 1.f;
                     tHit = -1.f;
@@ -456,11 +554,28 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
             next = min(end, next + (uint32_t)__popcll(idle));
         }
         if (!__any(active)) {
-            // chunk drained: take the next one
+            // a refill may have met only pixels past the image's edge
+            if (next < end) continue;
+            // chunk drained: take the next one.  The first fixedChunks belong
+            // to the launch's waves; the others are dealt to the queues in
+            // turn, a block draining its own.  Atomics on one counter queue up
+            // at 11 ns each (64 frames of 1280x720 in 16x16 chunks took 2.6 ms
+            // of them, 1.2 ms with eight counters 256 bytes apart), so a wave
+            // that finds the queue empty also tells its block.
             uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(queueCounter, 1u);
-            c = __shfl(c, 0, 64);
-            if (c >= totalChunks) break;
+            if (own) {
+                c = blockIdx.x * kWavesPerBlock + wave;
+                own = false;
+            } else {
+                if (fixedChunks >= totalChunks || *(volatile uint32_t *)&drained) break;
+                const uint32_t queue = blockIdx.x & (nQueues - 1);
+                if (lane == 0) c = atomicAdd(queueCounter + kSdfQueueStride * queue, 1u);
+                c = fixedChunks + __builtin_amdgcn_readfirstlane(c) * nQueues + queue;
+            }
+            if (c >= totalChunks) {
+                if (lane == 0) *(volatile uint32_t *)&drained = 1u;
+                break;
+            }
             job = ckd_find_job(jobs, nJobs, c, &SdfJob::chunkBase);
             const SdfJob &J = jobs[job];
             W = J.W;
@@ -471,62 +586,65 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
             const uint32_t local = c - J.chunkBase;
             cx0 = (local % J.chunksX) * kChunkSide;
             cy0 = (local / J.chunksX) * kChunkSide;
-            cw = min((uint32_t)kChunkSide, W - cx0);
-            cwM = ((1u << 20) + cw - 1) / cw;
-            const uint32_t chh = min((uint32_t)kChunkSide, H - cy0);
+            tilesX = (min((uint32_t)kChunkSide, W - cx0) + 7) / 8;
+            tilesM = ((1u << 20) + tilesX - 1) / tilesX;
             next = 0;
-            end = cw * chh;
+            end = 64 * tilesX * ((min((uint32_t)kChunkSide, H - cy0) + 7) / 8);
             bx = cam[0] - bound.x;
             by = cam[1] - bound.y;
             bz = cam[2] - bound.z;
-            // lane i stages sphere i; spheres past nSpheres become a neutral
-            // sphere whose distance is never the minimum (a centre 1e15 away
-            // from the camera, radius 0)
+            // the chunk's spheres: its corners' and its centre's rays (lanes
+            // 0-3 and the others) give the spread
+            uint32_t keep = sc.nSpheres >= 32 ? 0xffffffffu : (1u << sc.nSpheres) - 1u;
+            if (kChunkSide > 8) {
+                const uint32_t w = min((uint32_t)kChunkSide, W - cx0), h = min((uint32_t)kChunkSide, H - cy0);
+                const uint32_t x = cx0 + (lane < 4 ? (lane & 1) * (w - 1) : w >> 1);
+                const uint32_t y = cy0 + (lane < 4 ? (lane >> 1) * (h - 1) : h >> 1);
+                float ex, ey, ez;
+                ray_dir(cam, W, H, invH, x, y, ex, ey, ez);
+                const float mx = lane_f(ex, 4), my = lane_f(ey, 4), mz = lane_f(ez, 4);
+                const float vx = ex - mx, vy = ey - my, vz = ez - mz, v2 = vx * vx + vy * vy + vz * vz;
+                const float far2 = fmaxf(fmaxf(lane_f(v2, 0), lane_f(v2, 1)), fmaxf(lane_f(v2, 2), lane_f(v2, 3)));
+                const float spread = fmaf(1.01f, fsqrt(far2), 1e-5f);
+                keep = chunk_spheres(sc, cam, bound, bx, by, bz, mx, my, mz, spread, lane, keep);
+            }
+            // lane i stages sphere i, those kept packed to the front; the last
+            // group of four is filled up with a neutral sphere whose distance
+            // is never the minimum (a centre 1e15 away, radius 0)
+            sphGroups = (__popc(keep) + 3) / 4;
             if (lane < (uint32_t)kMaxSph) {
-                float r = 0.f, ox = 1e15f, oy = 0.f, oz = 0.f;
-                if ((int)lane < sc.nSpheres) {
-                    ox = cam[0] - sc.sphere[lane][0];
-                    oy = cam[1] - sc.sphere[lane][1];
-                    oz = cam[2] - sc.sphere[lane][2];
-                    r = sc.sphere[lane][3];
-                }
-                reinterpret_cast<float *>(&sphR[wave][lane >> 2])[lane & 3] = r;
-                sphOC[wave][lane] = f4{ox, oy, oz, 0.f};
+                reinterpret_cast<float *>(&sphR[wave][lane >> 2])[lane & 3] = 0.f;
+                sphOC[wave][lane] = f4{1e15f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (lane < (uint32_t)kMaxSph && (keep >> lane & 1u)) {
+                const uint32_t slot = __popc(keep & ((1u << lane) - 1u));
+                reinterpret_cast<float *>(&sphR[wave][slot >> 2])[slot & 3] = sc.sphere[lane][3];
+                sphOC[wave][slot] = f4{cam[0] - sc.sphere[lane][0], cam[1] - sc.sphere[lane][1],
+                                       cam[2] - sc.sphere[lane][2], 0.f};
             }
             __builtin_amdgcn_wave_barrier();
             continue;
         }
-        // march a few steps; the lanes' conditions are wave masks in SGPRs
+        // march a few steps; the lanes' conditions are wave masks in SGPRs.  A
+        // block whose lanes cannot reach the step limit does without its test.
         const float oyg = cam[1] - sc.groundY;
-        const float Rm = bound.w + 1e-3f;
-        const uint64_t activeM = __ballot(active);
-#pragma unroll
-        for (int k = 0; k < kStepsPerRefill; ++k) {
+        auto step = [&](auto limitTag) {
             const float t = tHit + d;
-            const uint64_t marchM = activeM & __builtin_amdgcn_fcmpf(d, sc.eps, kCmpGt) &
-                                    __builtin_amdgcn_sicmp(steps, sc.maxSteps, kCmpSlt) &
-                                    __builtin_amdgcn_fcmpf(t, sc.tMax, kCmpLt);
+            uint64_t marchM = __builtin_amdgcn_fcmpf(d, sc.eps, kCmpGt) & __builtin_amdgcn_fcmpf(t, sc.tMax, kCmpLt);
+            if constexpr (decltype(limitTag)::value) marchM &= __builtin_amdgcn_sicmp(steps, sc.maxSteps, kCmpSlt);
             float dist = fmaf(t, dy, oyg);
-            // Every sphere lies inside the bounding sphere (centre C, radius
-            // R), so each sphere's distance is at least |p - C| - R.  Where
-            // that bound exceeds the ground's distance by more than the
-            // rounding of either (1e-3 + 1e-3 |ground|, against errors of
-            // order 1e-5), no sphere can be the minimum: the ground's
-            // distance is the step, exactly as the full minimum gives it.
-            // The skip test is |p - C|^2 >= y^2 with y = ground + R +
-            // margin, without a square root: for y > 0 that is |p - C| >= y;
-            // for y <= 0 the test with the root skips too, and this one can
-            // only evaluate the spheres where it need not, which changes
-            // nothing.  The spheres are evaluated only when some marching
-            // lane needs them.
-            const float ub = t + Mb;
-            const float yb = fmaf(fabsf(dist), 1e-3f, dist + Rm);
-            const uint64_t nearM = __builtin_amdgcn_fcmpf(fmaf(ub, ub, E2b), yb * yb, kCmpLt);
+            // the spheres are evaluated only when some marching lane may need
+            // them (near_interval); elsewhere the ground's distance is the
+            // minimum, exactly as the loop would give it
+            const uint64_t nearM =
+                __builtin_amdgcn_fcmpf(t, tNear, kCmpGt) & __builtin_amdgcn_fcmpf(t, tFar, kCmpLt);
             if (marchM & nearM) {
                 evalSteps += (uint32_t)__popcll(marchM);
                 const uint32_t z = opaque_zero();
 #pragma unroll
-                for (int i = 0; i < kMaxSph / 4; ++i) {
+                for (int i = 0; i < kRegGroups; ++i) {
+                    if (i >= sphGroups) break;
                     const f4 r = sphR[wave][i + z];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
@@ -534,13 +652,33 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
                         dist = fminf(dist, fsqrt(fmaf(u, u, E2[4 * i + j])) - r[j]);
                     }
                 }
+                if constexpr (kMaxSph / 4 > kRegGroups) {
+#pragma unroll 1
+                    for (int i = kRegGroups; i < sphGroups; ++i) {
+                        const f4 r = sphR[wave][i];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            float m, e2;
+                            about_ray(sphOC[wave][4 * i + j], m, e2);
+                            const float u = t + m;
+                            dist = fminf(dist, fsqrt(fmaf(u, u, e2)) - r[j]);
+                        }
+                    }
+                }
             }
             tHit = sel_lane(marchM, t, tHit);
             d = sel_lane(marchM, dist, d);
             steps = add_lane(marchM, steps);
+        };
+        if (__ballot(active && steps > sc.maxSteps - kStepsPerRefill) == 0) {
+#pragma unroll
+            for (int k = 0; k < kStepsPerRefill; ++k) step(std::false_type{});
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < kStepsPerRefill; ++k) step(std::true_type{});
         }
-        // retire finished rays into the shade queue
         const float t = tHit + d;
+        // retire finished rays into the shade queue
         const bool fin = active && !(d > sc.eps && steps < sc.maxSteps && t < sc.tMax);
         const uint64_t finMask = __ballot(fin);
         if (finMask) {
@@ -550,6 +688,7 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
                 q[slot] = ShadeEntry{(uint32_t)job, xy, steps ? tHit : 0.f, t, dx, dy, dz, 0.f};
                 mySteps += (unsigned long long)steps;
                 active = false;
+                tHit = INFINITY;
             }
             qn += __popcll(finMask);
             __builtin_amdgcn_wave_barrier();
@@ -650,18 +789,18 @@ template <bool kHalf, int kMaxSph>
 void launch_persistent_steps(int steps, unsigned blocks, hipStream_t st, uint32_t *queueCounter,
                              uint32_t totalChunks, const SdfJob *jobs, int nJobs,
                              const ckd_sdf_scene &sc, unsigned long long *stepCount, uint32_t chunk,
-                             f4 bound, unsigned long long *work)
+                             uint32_t fixedChunks, uint32_t nQueues, bool own, f4 bound, unsigned long long *work)
 {
     if (steps <= 1)
-        k_sdf_persistent<kHalf, kMaxSph, 1><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, work);
+        k_sdf_persistent<kHalf, kMaxSph, 1><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, work);
     else if (steps == 2)
-        k_sdf_persistent<kHalf, kMaxSph, 2><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, work);
+        k_sdf_persistent<kHalf, kMaxSph, 2><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, work);
     else if (steps == 4)
-        k_sdf_persistent<kHalf, kMaxSph, 4><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, work);
+        k_sdf_persistent<kHalf, kMaxSph, 4><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, work);
     else if (steps == 8)
-        k_sdf_persistent<kHalf, kMaxSph, 8><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, work);
+        k_sdf_persistent<kHalf, kMaxSph, 8><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, work);
     else
-        k_sdf_persistent<kHalf, kMaxSph, 16><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, work);
+        k_sdf_persistent<kHalf, kMaxSph, 16><<<blocks, 256, 0, st>>>(queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, work);
 }
 
 // A sphere containing every sphere of the scene: centre the centroid of the
@@ -689,20 +828,32 @@ f4 bounding_sphere(const ckd_sdf_scene &sc)
     return f4{fx, fy, fz, std::nextafter((float)R, 3.4e38f)};
 }
 
-ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t totalChunks,
+// The side of the batch's chunks, at most the tuned one.  Small chunks spread a
+// small batch over the chip (at least as many chunks as resident waves); large
+// ones refill lanes longer and find the chunk's spheres less often (8x8 ones
+// not at all, which a scene of many spheres pays for).  Measured, us, sides 8,
+// 16, 32: 8 spheres 1280x720, 1 frame 44, 60, 148; 4 frames 124, 113, 182; 16
+// frames 466, 311, 359; 32 frames 935, 590, 614; 64 frames 1830, 1122, 1101; 32
+// spheres 2560x1440, 2 frames -, 338, 567; 24 frames -, 3056, 2962.
+uint32_t sdf_chunk_side(int tuned, size_t pixels, int nSpheres)
+{
+    const uint32_t side = pixels <= 2u << 20 && nSpheres <= 8 ? 8 : pixels <= 32u << 20 ? 16 : 32;
+    return std::min(side, (uint32_t)tuned);
+}
+
+ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t totalChunks, uint32_t chunk,
                                  const SdfJob *jobs, int nJobs, const ckd_sdf_scene &sc,
                                  int shading, unsigned long long *stepCount, bool helper, bool alone)
 {
     if (totalChunks == 0) return CKD_OK;
     const bool big = sc.nSpheres > 8;
     const int steps = ctx->tuning.sdfStepsPerRefill;
-    const uint32_t chunk = (uint32_t)ctx->tuning.sdfChunk;
     // persistent: sdfBlocksPerCU 4-wave blocks per CU; surplus blocks find
     // the queue empty and exit.  A helper launch (the batch's second stream,
     // once its voxel and tunnel work is done) adds the blocks that fill each
     // CU up to the kernel's occupancy and drains the same queue.  A batch
-    // with nothing beside the march (alone) gets at least that occupancy:
-    // the tuned count leaves room for work that is not there.
+    // with nothing beside the march (alone) gets that occupancy: the tuned
+    // count leaves room for work that is not there.
     int perCU = ctx->tuning.sdfBlocksPerCU;
     const int fit = shading == CKD_SHADE_FP16
                         ? (big ? persistent_blocks_per_cu<true, 32>(steps) : persistent_blocks_per_cu<true, 8>(steps))
@@ -710,22 +861,28 @@ ckd_status launch_sdf_persistent(ckd_ctx *ctx, uint32_t *queueCounter, uint32_t 
     if (helper) {
         perCU = fit - perCU;
         if (perCU <= 0) return CKD_OK;
-    } else if (alone && perCU < fit) {
+    } else if (alone && fit > 0) {
         perCU = fit;
     }
     unsigned blocks = (unsigned)ctx->cuCount * (unsigned)perCU;
     const unsigned useful = (totalChunks + kWavesPerBlock - 1) / kWavesPerBlock;
     if (blocks > useful) blocks = useful;
     if (blocks == 0) blocks = 1;
+    // with nothing beside the march every block is resident: each wave's first
+    // chunk is its own
+    const bool own = alone;
+    // a queue needs a block of the main launch to drain it
+    const uint32_t nQueues = blocks >= kSdfQueues ? kSdfQueues : 1;
+    const uint32_t fixedChunks = alone ? std::min(totalChunks, (uint32_t)(blocks * kWavesPerBlock)) : 0u;
     // only the main launch is timed: it spans the whole march of the batch
     const f4 bound = bounding_sphere(sc);
     KernelTimer kt(ctx, helper ? -1 : CKD_KT_SDF_PERSISTENT);
     if (shading == CKD_SHADE_FP16) {
-        if (big) launch_persistent_steps<true, 32>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, ctx->sdfWork);
-        else launch_persistent_steps<true, 8>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, ctx->sdfWork);
+        if (big) launch_persistent_steps<true, 32>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, ctx->sdfWork);
+        else launch_persistent_steps<true, 8>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, ctx->sdfWork);
     } else {
-        if (big) launch_persistent_steps<false, 32>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, ctx->sdfWork);
-        else launch_persistent_steps<false, 8>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, bound, ctx->sdfWork);
+        if (big) launch_persistent_steps<false, 32>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, ctx->sdfWork);
+        else launch_persistent_steps<false, 8>(steps, blocks, ctx->stream, queueCounter, totalChunks, jobs, nJobs, sc, stepCount, chunk, fixedChunks, nQueues, own, bound, ctx->sdfWork);
     }
     return check_launch("sdf persistent");
 }

@@ -241,10 +241,10 @@ CKD_API ckd_status ckd_sdf_render(ckd_ctx *ctx, uint32_t *dst, unsigned W,
 
 /* Measurement hook, no reference counterpart: while counters (device memory,
  * two u64) is non-null, the batched SDF kernel adds to counters[0] the march
- * steps that evaluated the spheres and to counters[1] the shaded pixels
- * whose normal evaluated them.  The others took the ground's distance after
- * a bounding-sphere test showed no sphere could be nearer (the result is the
- * same either way).  NULL switches it off. */
+ * steps that evaluated spheres (those that can be the nearest surface in the
+ * step's chunk) and to counters[1] the shaded pixels whose normal evaluated
+ * them.  The others took the ground's distance after a bounding-sphere test
+ * showed no sphere could be nearer (the result is the same either way).  NULL switches it off. */
 CKD_API ckd_status ckd_sdf_work_counter(ckd_ctx *ctx, unsigned long long *counters);
 
 /* ---- tunnel frame (no reference counterpart as a whole: the tunnel
@@ -292,7 +292,8 @@ typedef struct ckd_request {
 typedef struct ckd_tuning {
     int sdfStepsPerRefill; /* march steps between lane refills: 1, 2, 4, 8
                               or 16                                         */
-    int sdfChunk;          /* side of the square pixel chunks: 16 or 32     */
+    int sdfChunk;          /* largest side of the square pixel chunks: 16 or
+                              32 (small batches take smaller ones)         */
     int sdfBlocksPerCU;    /* persistent 4-wave blocks per CU: 1..32 while
                               voxel or tunnel work runs beside the march; a
                               batch of SDF requests only gets at least the
@@ -312,7 +313,7 @@ CKD_API ckd_status ckd_set_tuning(ckd_ctx *ctx, const ckd_tuning *t);
  * given shading precision, VOXEL requests the landscape maps, TUNNEL
  * requests `tex` (2^texLog2 square) and need scratch: tmp (device) of at
  * least sum over TUNNEL requests of W*H pixels.  stepCount as above.
- * SDF requests run in one persistent launch over a queue of 32x32-pixel
+ * SDF requests run in one persistent launch over queues of square pixel
  * chunks, VOXEL requests in one launch, TUNNEL requests in two. */
 CKD_API ckd_status ckd_render_batch(ckd_ctx *ctx, const ckd_request *requests,
                                     unsigned n, const ckd_sdf_scene *scene,
