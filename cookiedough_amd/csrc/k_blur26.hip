@@ -3,30 +3,30 @@
 // HorzBlur32 (code/boxblur.cpp:87-212) keeps a running i32 sum per channel
 // that adds the lerp term T(j) = p[j] + (((p[j+1]-p[j])*alpha) >> 16) at
 // the head and subtracts it at the tail.  Integer addition is associative,
-// so the sum at output o has the closed form
-//   S(o) = S0 + sum_{j=iSpan+1}^{min(iSpan+o, L)} T(j) - sum_{j<max(o-iSpan,0)} T(j)
-//   S0   = sum_{j<iSpan} p[j] + ((p[iSpan]*alpha) >> 16)
-// and each pass becomes prefix sums over T in LDS, one block per line.  The
-// reference reads p[L] and p[L+1] past every line: the next line's first
-// pixels, or (after the last line) two pixels defined here as zero.
+// so the sums of a line's outputs are a prefix sum of what each one adds,
+//   S(o) = S0 - T(iSpan) + sum_{o'<=o} (T(o'+iSpan) - T(o'-iSpan-1)),
+//   S0   = sum_{j<iSpan} p[j] + ((p[iSpan]*alpha) >> 16),
+// with T zero before the line and after T(L).  The reference reads p[L] and
+// p[L+1] past every line: the next line's first pixels, or (after the last
+// line) two pixels defined here as zero.
 // Output: iDiv (mul_epu32 of the low dword, >> 22, hadd of the two halves)
 // and v2cISSE32 (code/boxblur.cpp:69-79, code/util.h:152-154).
 #include "ckd_internal.h"
 #include "ckd_pixel.h"
 
-#include <cstring>
+#include <algorithm>
 
 namespace {
 
-constexpr int kMaxRes = 2048, kMaxRadius = 500, kBlock = 256;
+constexpr int kMaxRes = 2048, kMaxRadius = 500, kMaxWaves = 16;
 
 struct B26Params {
     int32_t iSpan, iAlpha;
-    uint32_t iScale; // low dword of the 10:22 scale (what _mm_mul_epu32 uses)
-    uint32_t spanScales[kMaxRadius];
+    uint32_t iScale; // the 10:22 scale
+    float halfScale, dScale;
 };
 
-// code/boxblur.cpp:98-124, host FP32 without contraction
+// code/boxblur.cpp:98-124, FP32 without contraction
 #pragma clang fp contract(off)
 void b26_setup(unsigned xRes, float strength, float gain, B26Params &P)
 {
@@ -39,148 +39,294 @@ void b26_setup(unsigned xRes, float strength, float gain, B26Params &P)
     P.iSpan = (int32_t)iSpan;
     P.iScale = (uint32_t)(uint64_t)(int64_t)(scale * (float)(1 << 22));
     P.iAlpha = (int32_t)(65536.f * alpha);
-    const float halfScale = scale * 0.5f;
-    const float dScale = halfScale / (float)iSpan;
-    memset(P.spanScales, 0, sizeof(P.spanScales));
-    for (unsigned i = 0; i < iSpan; ++i)
-        P.spanScales[i] = (uint32_t)(uint64_t)(int64_t)((halfScale + (float)i * dScale) * (float)(1 << 22));
+    P.halfScale = scale * 0.5f;
+    P.dScale = iSpan ? P.halfScale / (float)iSpan : 0.f;
+}
+
+// the scale of an output i < iSpan pixels from either end of its line
+CKD_DEV uint32_t span_scale(float halfScale, float dScale, int i)
+{
+    return (uint32_t)((halfScale + (float)i * dScale) * (float)(1 << 22));
 }
 #pragma clang fp contract(on)
 
-CKD_DEV int32_t lerp_term(int32_t A, int32_t B, int32_t alpha)
-{
-    return A + ((int32_t)((uint32_t)(B - A) * (uint32_t)alpha) >> 16);
-}
+// One launch: `passes` passes over every line, then the store.
+struct B26Launch {
+    int32_t L, rows, passes;
+    int32_t iSpan;
+    uint32_t weights, round; // lerp_terms
+    uint32_t scale;          // iScale << scaleShift
+    int32_t sumShift, scaleShift;
+    float halfScale, dScale;
+    int32_t colStride, rowStride; // output o of line r: r * colStride + o * rowStride
+    int32_t lines, wavesPerLine, haloWaves, blocks;
+};
 
-// two channels (c, c+2 of byte order B,G,R,A -> fields lo/hi) per u64; the
-// prefix sums of T stay below 2^32 per field, so fields never carry
-CKD_DEV uint64_t pack2(int32_t lo, int32_t hi) { return (uint64_t)(uint32_t)lo | ((uint64_t)(uint32_t)hi << 32); }
+// Four channels' values of at most 16 bits: B and R (even), G and A (odd), each
+// two as hi * 65536 + lo.  Such pairs add and subtract as one number, a negative
+// lo borrowing from hi.
+struct Pairs {
+    uint32_t even, odd;
+};
+CKD_DEV Pairs pairs_of(uint32_t pixel) { return {pixel & 0x00ff00ffu, ckd_perm(0, pixel, 0x0c030c01u)}; }
+CKD_DEV int32_t pair_lo(uint32_t v) { return (int32_t)(int16_t)v; }
+CKD_DEV int32_t pair_hi(uint32_t v) { return (int32_t)(v + 0x8000u) >> 16; }
 
-CKD_DEV uint32_t div_lane(int32_t sum, uint32_t k)
+// The lerp terms of neighbours a, b:
+//   A + (((B - A) * alpha) >> 16) = (A * (65536 - alpha) + B * alpha) >> 16,
+// one dot product; alpha = 0 takes weights 65535, 0 and 65535 more, which gives
+// A as well (65536 does not fit the weight's 16 bits).
+CKD_DEV Pairs lerp_terms(uint32_t a, uint32_t b, uint32_t weights, uint32_t round)
 {
-    const uint64_t r = ((uint64_t)(uint32_t)sum * (uint64_t)k) >> 22;
-    const int32_t lane = (int32_t)((uint32_t)r + (uint32_t)(r >> 32));
-    const int32_t u16 = lane < 0 ? 0 : (lane > 65535 ? 65535 : lane);
-    const int32_t s16 = (int32_t)(int16_t)(uint16_t)u16;
-    return (uint32_t)(s16 < 0 ? 0 : (s16 > 255 ? 255 : s16));
-}
-
-// inclusive block scan of a pair of u64 values (256 threads, 4 waves)
-CKD_DEV void block_scan2(uint64_t &a, uint64_t &b, uint64_t *sh /* 8 entries */)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+    const us2 w = __builtin_bit_cast(us2, weights);
+    uint32_t t[4];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint64_t ya = __shfl_up(a, o, 64);
-        const uint64_t yb = __shfl_up(b, o, 64);
-        if (lane >= o) {
-            a += ya;
-            b += yb;
+    for (int c = 0; c < 4; ++c)
+        t[c] = __builtin_amdgcn_udot2(__builtin_bit_cast(us2, ckd_perm(b, a, 0x0c040c00u + 0x00010001u * c)), w,
+                                      round, false);
+    return {ckd_perm(t[2], t[0], 0x0c060c02u), ckd_perm(t[3], t[1], 0x0c060c02u)};
+}
+
+template <int kCtrl, int kRows> CKD_DEV int32_t dpp_sum(int32_t v)
+{
+    return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
+}
+
+// sums over the lanes of a row (16) up to each one's, of the rows up to each one
+CKD_DEV int32_t row_scan(int32_t v)
+{
+    v = dpp_sum<0x111, 0xf>(v); // row_shr:1, 2, 4, 8
+    v = dpp_sum<0x112, 0xf>(v);
+    v = dpp_sum<0x114, 0xf>(v);
+    return dpp_sum<0x118, 0xf>(v);
+}
+CKD_DEV int32_t rows_scan(int32_t v)
+{
+    return dpp_sum<0x143, 0xc>(dpp_sum<0x142, 0xa>(v)); // row_bcast:15, 31
+}
+
+// lo * m + c and hi * m + c of a pair whose lo is not negative
+CKD_DEV int32_t mad_lo(uint32_t v, int32_t m, int32_t c)
+{
+    int32_t r;
+    asm("v_mad_i32_i16 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(m), "v"(c));
+    return r;
+}
+CKD_DEV int32_t mad_hi(uint32_t v, int32_t m, int32_t c)
+{
+    int32_t r;
+    asm("v_mad_i32_i16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(r) : "v"(v), "s"(m), "v"(c));
+    return r;
+}
+// (a * b) >> 32 of a, b of 24 bits with the sign
+CKD_DEV uint32_t mul_hi24(int32_t a, uint32_t b)
+{
+    uint32_t r;
+    asm("v_mul_hi_i32_i24 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+typedef int32_t i4 __attribute__((ext_vector_type(4)));
+
+// Sums of the lanes' pairs up to each lane, B G R A, of values that kPer pixels
+// give: over a row as pairs, as long as 16 lanes' fit those.
+constexpr uint32_t kBias = 0x1000; // above what a lane's sums go below 0
+template <int kPer> CKD_DEV i4 wave_sums(Pairs p)
+{
+    i4 s;
+    if constexpr (16 * kPer * 255 <= 32767) {
+        const uint32_t even = row_scan(p.even), odd = row_scan(p.odd);
+        s = i4{pair_lo(even), pair_lo(odd), pair_hi(even), pair_hi(odd)};
+    } else {
+        s = i4{row_scan(pair_lo(p.even)), row_scan(pair_lo(p.odd)), row_scan(pair_hi(p.even)),
+               row_scan(pair_hi(p.odd))};
+    }
+    return i4{rows_scan(s.x), rows_scan(s.y), rows_scan(s.z), rows_scan(s.w)};
+}
+
+// A block blurs P.lines lines, P.passes times, a line on P.wavesPerLine waves
+// with kPer consecutive pixels on a lane; pixels stay in registers from pass to
+// pass.  A pass writes the line's T to LDS with zeros either side, sums
+// T(o+iSpan) - T(o-iSpan-1) over the lane, the wave (DPP) and the line's waves,
+// and scales.  kPer is odd: lanes that far apart hit all banks.
+//
+// The reads past a line's end couple the lines: pass q of the block's last line
+// needs two pixels of the next line after pass q - 1.  haloWaves more waves carry
+// that line's first pixels along (as many as the passes left need: two for one
+// pass, iSpan + 1 more for each further one).
+//
+// A pass is bound by its three barriers' chains and the VALU (half busy): 4.7 us
+// of 1920x1080, and 5.7 us for the loads and stores of a launch (3.2 us at the
+// copy's rate).  Against a launch a pass with the prefix sums in LDS: 59 -> 20 us
+// for three passes along the rows, 63 -> 27 along the columns.
+template <int kPer>
+__global__ __launch_bounds__(64 * kMaxWaves, kPer <= 7 ? 8 : 6)
+void k_b26_lines(uint32_t *__restrict__ out, const uint32_t *__restrict__ in, const B26Launch P)
+{
+    extern __shared__ Pairs lds[];
+    // per wave and channel: the sum of the differences, the share of S0 - T(iSpan)
+    __shared__ int32_t totals[4 * kMaxWaves], starts[4 * kMaxWaves];
+    __shared__ uint32_t firsts[kMaxWaves + 1], seconds[kMaxWaves + 1]; // pixels 0 and 1 of each wave's
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int perXcd = (P.blocks + 7) >> 3, block = (blockIdx.x & 7) * perXcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= perXcd || block >= P.blocks) return;
+
+    const int L = P.L, iSpan = P.iSpan, nw = P.wavesPerLine;
+    const int slot = min(wave / nw, P.lines), w = wave - slot * nw, slotWaves = slot < P.lines ? nw : P.haloWaves;
+    const int row = block * P.lines + slot;
+    const bool halo = slot == P.lines, last = !halo && w == nw - 1;
+    const int reach = nw * 64 * kPer, stride = reach + 2 * iSpan + 2;
+    const int base = w * 64 * kPer, j0 = base + lane * kPer; // the lane's first pixel
+    Pairs *T = lds + slot * stride + iSpan + 1;              // T[0]: of pixel 0
+
+    for (int i = w * 64 + lane; i <= iSpan; i += slotWaves * 64) T[i - iSpan - 1] = {0, 0};
+    if (!halo)
+        for (int i = L + 1 + w * 64 + lane; i <= reach + iSpan; i += slotWaves * 64) T[i] = {0, 0};
+    if (base > iSpan && lane < 4) starts[4 * wave + lane] = 0;
+
+    // the line's pixels, and the two after it (last wave)
+    const int n = L * P.rows, at = row * L + j0;
+    uint32_t px[kPer + 1], after0 = 0, after1 = 0;
+#pragma unroll
+    for (int i = 0; i <= kPer; ++i) {
+        const uint32_t v = in[min(at + i, n - 1)];
+        px[i] = at + i < n ? v : 0u;
+    }
+    if (last && row + 1 < P.rows) {
+        after0 = in[(row + 1) * L];
+        after1 = in[(row + 1) * L + 1];
+    }
+
+    const int32_t sumUnit = 1 << P.sumShift;
+    const int sumLane = 4 * (wave - w) + lane; // lane 4 v + c: channel c of the line's wave v
+    for (int pass = 0;; ++pass) {
+        const bool store = pass == P.passes - 1, live = !(halo && store);
+        if (live) {
+            Pairs t[kPer];
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) t[i] = lerp_terms(px[i], px[i + 1], P.weights, P.round);
+            if (last) {
+#pragma unroll
+                for (int i = 0; i < kPer; ++i)
+                    if (j0 + i < L) T[j0 + i] = t[i];
+                if (lane == 0) T[L] = lerp_terms(after0, after1, P.weights, P.round);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) T[j0 + i] = t[i];
+            }
+            if (base <= iSpan) {
+                Pairs sum = {0, 0}, edgeT = {0, 0};
+                uint32_t edge = 0;
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const Pairs p = pairs_of(j0 + i < iSpan ? px[i] : 0u);
+                    sum.even += p.even;
+                    sum.odd += p.odd;
+                    if (j0 + i == iSpan) {
+                        edge = px[i];
+                        edgeT = t[i];
+                    }
+                }
+                // (p * alpha) >> 16: the term between 0 and p
+                const Pairs frac = lerp_terms(0, edge, P.weights & 0xffff0000u, 0);
+                sum.even += frac.even - edgeT.even;
+                sum.odd += frac.odd - edgeT.odd;
+                const i4 s = wave_sums<kPer>(sum);
+                if (lane == 63) *reinterpret_cast<i4 *>(starts + 4 * wave) = s;
+            }
+        }
+        __syncthreads();
+        // the lane's prefix sums, lo biased to stay positive, and the wave's
+        uint32_t even[kPer], odd[kPer];
+        i4 upTo;
+        if (live) {
+            Pairs s = {kBias, kBias};
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                const Pairs h = T[j0 + i + iSpan], l = T[j0 + i - iSpan - 1];
+                even[i] = s.even += h.even - l.even;
+                odd[i] = s.odd += h.odd - l.odd;
+            }
+            upTo = wave_sums<kPer>({s.even - kBias, s.odd - kBias});
+            if (lane == 63) *reinterpret_cast<i4 *>(totals + 4 * wave) = upTo;
+        }
+        __syncthreads();
+        if (live) {
+            // S0 - T(iSpan) and the sums of the waves before: four waves a row
+            int32_t part = 0;
+            if (lane < 4 * slotWaves) part = starts[sumLane];
+            if (lane < 4 * w) part += totals[sumLane];
+            part = dpp_sum<0x118, 0xf>(dpp_sum<0x114, 0xf>(part)); // row_shr:4, 8
+            i4 line = {0, 0, 0, 0};
+            for (int v = 0; v < slotWaves; v += 4)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) line[c] += __builtin_amdgcn_readlane(part, 4 * v + 12 + c);
+            // less the lane's own, which its prefix sums add again
+            i4 before = (upTo + line) << P.sumShift;
+            before.x = mad_lo(even[kPer - 1], -sumUnit, before.x);
+            before.y = mad_lo(odd[kPer - 1], -sumUnit, before.y);
+            before.z = mad_hi(even[kPer - 1], -sumUnit, before.z);
+            before.w = mad_hi(odd[kPer - 1], -sumUnit, before.w);
+            uint32_t scale[kPer];
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) scale[i] = P.scale;
+            if (base < iSpan || base + 64 * kPer > L - iSpan)
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const int o = j0 + i, fromEnd = o < iSpan ? o : L - 1 - o;
+                    if (fromEnd < iSpan) scale[i] = span_scale(P.halfScale, P.dScale, fromEnd) << P.scaleShift;
+                }
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                // a negative sum gives a negative product, which is taken as 0
+                const uint32_t b = mul_hi24(mad_lo(even[i], sumUnit, before.x), scale[i]);
+                const uint32_t g = mul_hi24(mad_lo(odd[i], sumUnit, before.y), scale[i]);
+                const uint32_t r = mul_hi24(mad_hi(even[i], sumUnit, before.z), scale[i]);
+                const uint32_t a = mul_hi24(mad_hi(odd[i], sumUnit, before.w), scale[i]);
+                px[i] = ckd_perm(ckd_sat_pk_u8(ckd_perm(a, r, 0x05040100u)),
+                                 ckd_sat_pk_u8(ckd_perm(g, b, 0x05040100u)), 0x05040100u);
+            }
+        }
+        if (store) break;
+        if (row >= P.rows)
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) px[i] = 0;
+        if (lane == 0) {
+            firsts[wave] = px[0];
+            seconds[wave] = px[1];
+        }
+        __syncthreads();
+        // the pixels after the lane's and after the line's
+        const uint32_t next = firsts[wave + 1];
+        px[kPer] = __builtin_amdgcn_update_dpp(next, px[0], 0x130, 0xf, 0xf, false); // wave_shl:1
+        if (last) {
+            after0 = next;
+            after1 = seconds[wave + 1];
+#pragma unroll
+            for (int i = 0; i <= kPer; ++i)
+                if (j0 + i == L) px[i] = after0;
         }
     }
-    if (lane == 63) {
-        sh[wave] = a;
-        sh[4 + wave] = b;
+
+    // to LDS, to be stored in the order of the output's addresses
+    uint32_t *staged = reinterpret_cast<uint32_t *>(lds);
+    if (!halo) {
+        uint32_t *stage = staged + slot * reach + j0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) stage[i] = px[i];
     }
     __syncthreads();
-    for (int w = 0; w < wave; ++w) {
-        a += sh[w];
-        b += sh[4 + w];
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_b26_pass(uint32_t *__restrict__ out,
-                                                     const uint32_t *__restrict__ in, int L,
-                                                     int rows, int colStride, int rowStride,
-                                                     B26Params P)
-{
-    extern __shared__ uint64_t lds[];
-    uint64_t *PT0 = lds;                 // L+2 prefix sums, channels B,R
-    uint64_t *PT1 = lds + (L + 2);       // L+2 prefix sums, channels G,A
-    uint32_t *px = reinterpret_cast<uint32_t *>(lds + 2 * (L + 2)); // L+2 pixels
-    __shared__ uint64_t scanSh[8];
-    __shared__ int32_t s0Sh[4][4];
-
-    const int row = blockIdx.x;
-    const size_t n = (size_t)L * rows;
-    const size_t base = (size_t)row * L;
-    for (int i = threadIdx.x; i < L + 2; i += kBlock)
-        px[i] = (base + i < n) ? in[base + i] : 0u;
-    __syncthreads();
-
-    const int iSpan = P.iSpan, alpha = P.iAlpha;
-    // T(j), j in [0, L], prefix over chunks
-    const int nT = L + 1;
-    const int chunk = (nT + kBlock - 1) / kBlock;
-    const int c0 = threadIdx.x * chunk, c1 = min(c0 + chunk, nT);
-    uint64_t l0 = 0, l1 = 0;
-    int32_t s0[4] = {0, 0, 0, 0};
-    for (int j = c0; j < c1; ++j) {
-        const uint32_t a = px[j], b = px[j + 1];
-        int32_t t[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            t[k] = lerp_term((int32_t)((a >> (8 * k)) & 0xff), (int32_t)((b >> (8 * k)) & 0xff), alpha);
-        l0 += pack2(t[0], t[2]);
-        l1 += pack2(t[1], t[3]);
-    }
-    // S0 partial sums over p[j < iSpan] (any thread's chunk of pixels)
-    for (int j = threadIdx.x; j < iSpan; j += kBlock) {
-        const uint32_t a = px[j];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s0[k] += (int32_t)((a >> (8 * k)) & 0xff);
-    }
-    uint64_t i0 = l0, i1 = l1;
-    block_scan2(i0, i1, scanSh);
-    uint64_t run0 = i0 - l0, run1 = i1 - l1;
-    if (threadIdx.x == 0) PT0[0] = PT1[0] = 0;
-    for (int j = c0; j < c1; ++j) {
-        const uint32_t a = px[j], b = px[j + 1];
-        int32_t t[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            t[k] = lerp_term((int32_t)((a >> (8 * k)) & 0xff), (int32_t)((b >> (8 * k)) & 0xff), alpha);
-        run0 += pack2(t[0], t[2]);
-        run1 += pack2(t[1], t[3]);
-        PT0[j + 1] = run0;
-        PT1[j + 1] = run1;
-    }
-    // reduce S0 over the block
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        int32_t v = s0[k];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if ((threadIdx.x & 63) == 0) s0Sh[threadIdx.x >> 6][k] = v;
-    }
-    __syncthreads();
-    int32_t S0[4];
-    {
-        const uint32_t a = px[iSpan];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            S0[k] = s0Sh[0][k] + s0Sh[1][k] + s0Sh[2][k] + s0Sh[3][k];
-            S0[k] += (int32_t)((uint32_t)((a >> (8 * k)) & 0xff) * (uint32_t)alpha) >> 16;
-        }
-    }
-    const uint64_t Hbase0 = PT0[iSpan + 1], Hbase1 = PT1[iSpan + 1];
-    for (int o = threadIdx.x; o < L; o += kBlock) {
-        const int hEnd = min(iSpan + o, L) + 1;
-        const int tEnd = max(o - iSpan, 0);
-        // heads minus tails can be negative, so subtract field by field (a
-        // u64 difference would borrow across the 32-bit fields)
-        const uint64_t a0 = PT0[hEnd], a1 = PT1[hEnd], t0 = PT0[tEnd], t1 = PT1[tEnd];
-        const int32_t sum[4] = {
-            S0[0] + (int32_t)((uint32_t)a0 - (uint32_t)Hbase0 - (uint32_t)t0),
-            S0[1] + (int32_t)((uint32_t)a1 - (uint32_t)Hbase1 - (uint32_t)t1),
-            S0[2] + (int32_t)((uint32_t)(a0 >> 32) - (uint32_t)(Hbase0 >> 32) - (uint32_t)(t0 >> 32)),
-            S0[3] + (int32_t)((uint32_t)(a1 >> 32) - (uint32_t)(Hbase1 >> 32) - (uint32_t)(t1 >> 32))};
-        const uint32_t k = o < iSpan ? P.spanScales[o]
-                                     : (o >= L - iSpan ? P.spanScales[L - 1 - o] : P.iScale);
-        uint32_t pix = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) pix |= div_lane(sum[c], k) << (8 * c);
-        out[(size_t)row * colStride + (size_t)o * rowStride] = pix;
+    if (P.rowStride == 1) {
+        if (!halo && row < P.rows)
+            for (int o = w * 64 + lane; o < L; o += nw * 64)
+                out[(size_t)row * P.colStride + o] = staged[slot * reach + o];
+    } else {
+        const int shift = P.lines - 1, g = threadIdx.x & shift; // one or two lines
+        const int r = block * P.lines + g;
+        if (r < P.rows)
+            for (int o = threadIdx.x >> shift; o < L; o += blockDim.x >> shift)
+                out[(size_t)r * P.colStride + (size_t)o * P.rowStride] = staged[g * reach + o];
     }
 }
 
@@ -202,33 +348,111 @@ __global__ __launch_bounds__(256) void k_transpose(uint32_t *__restrict__ dst,
     }
 }
 
+// How a launch covers the lines.
+//
+// per, the pixels of a lane: what a line's waves cost is linear in it (a scan of
+// the wave and the exchange, about three pixels' worth), so it follows from how
+// the line divides, except where all waves fit the chip at once: then the least,
+// for the shortest chain (320x180, 2 passes both ways: 9.7 us with 3, 11.0 with 5).
+// Three passes of 1920x1080: along the rows 20.0 us with 5, 21.8 with 7, 24.5 with
+// 3; along the columns 28.1 with 9 or 7, 30.9 with 5.
+// lines: two a block give a transposed store 8-byte pieces (26.7 us instead of
+// 28.1), where there are blocks enough left; otherwise blocks of one line fill
+// the chip more evenly (1080 lines: 20.0 us, 22.8 with two).
+// passes: as many as a halo of a quarter of its waves allows (three of 1920x1080:
+// 20.0 us in one launch, 34.8 in three).
+struct B26Shape {
+    int per, wavesPerLine, lines, haloWaves, passes;
+};
+
+// the lines' T, a margin of iSpan + 1 either side of each
+size_t b26_lds(int per, int waves, int lines, int iSpan)
+{
+    return ((size_t)waves * 64 * per + (size_t)(lines + 1) * (2 * iSpan + 2)) * sizeof(Pairs);
+}
+
+B26Shape b26_shape(int L, int rows, int iSpan, int passes, bool transposed)
+{
+    B26Shape s = {};
+    auto line_waves = [L](int per) { return (int)ckd_div_up((unsigned)L, 64u * per); };
+    s.per = 3;
+    if (rows * line_waves(3) > 2048)
+        for (int per = 5; per <= 9; per += 2)
+            if (line_waves(per) * (per + 3) < line_waves(s.per) * (s.per + 3)) s.per = per;
+    s.wavesPerLine = line_waves(s.per);
+    s.lines = transposed && rows >= 1536 && s.wavesPerLine <= 6
+                      && b26_lds(s.per, 2 * s.wavesPerLine, 2, iSpan) <= 65536 ? 2 : 1;
+    const int most = s.lines * s.wavesPerLine;
+    s.passes = 1;
+    for (int f = 2; f <= passes; ++f) {
+        const int need = (f - 1) * (iSpan + 1) + 1; // pixels of the next line
+        const int waves = (int)ckd_div_up((unsigned)need, 64u * s.per);
+        if (need > L || waves > (most + 3) / 4 || most + waves > kMaxWaves
+            || b26_lds(s.per, most + waves, s.lines, iSpan) > 65536)
+            break;
+        s.passes = f;
+        s.haloWaves = waves;
+    }
+    return s;
+}
+
+template <int kPer>
+void launch_lines(ckd_ctx *ctx, uint32_t *out, const uint32_t *in, const B26Launch &P)
+{
+    const int waves = P.lines * P.wavesPerLine + P.haloWaves;
+    const size_t lds = b26_lds(kPer, waves, P.lines, P.iSpan);
+    k_b26_lines<kPer><<<(P.blocks + 7) / 8 * 8, 64 * waves, lds, ctx->stream>>>(out, in, P);
+}
+
 // HorzBlur32's pass loop (code/boxblur.cpp:126-211) over device buffers
 ckd_status horz(ckd_ctx *ctx, uint32_t *pDest, uint32_t *pScratch, const uint32_t *pSrc,
                 unsigned xRes, unsigned yRes, unsigned wCol, unsigned wRow, float strength,
                 float gain, unsigned numPasses)
 {
-    B26Params P;
-    b26_setup(xRes, strength, gain, P);
+    B26Params B;
+    b26_setup(xRes, strength, gain, B);
+    B26Launch P = {};
+    P.L = (int)xRes;
+    P.rows = (int)yRes;
+    P.iSpan = B.iSpan;
+    P.weights = B.iAlpha ? (uint32_t)(65536 - B.iAlpha) | (uint32_t)B.iAlpha << 16 : 65535u;
+    P.round = B.iAlpha ? 0u : 65535u;
+    P.halfScale = B.halfScale;
+    P.dScale = B.dScale;
+    // (sum * scale) >> 22 as the high half of a product of 24-bit factors with
+    // signs, 10 bits shared out between them: a sum is at most (2 iSpan + 2) * 255
+    // and a scale at most 2^22 / (iSpan + 1), so the two always fit
+    int sumBits = 0;
+    while (((2 * B.iSpan + 2) * 255) >> sumBits) ++sumBits;
+    P.sumShift = std::min(10, 23 - sumBits);
+    P.scaleShift = 10 - P.sumShift;
+    P.scale = B.iScale << P.scaleShift;
+
+    unsigned launches = 0;
+    for (unsigned left = numPasses; left; ++launches)
+        left -= (unsigned)b26_shape(P.L, P.rows, P.iSpan, (int)left, wRow != 1).passes;
     const uint32_t *pRead = pSrc;
-    if ((numPasses & 1) == 0) {
-        uint32_t *t = pDest;
-        pDest = pScratch;
-        pScratch = t;
-    }
-    const size_t lds = (size_t)(xRes + 2) * 2 * sizeof(uint64_t) + (size_t)(xRes + 2) * sizeof(uint32_t);
-    for (unsigned pass = 0; pass < numPasses; ++pass) {
-        int cs = (int)xRes, rs = 1;
-        if (pass == numPasses - 1) {
-            cs = (int)wCol;
-            rs = (int)wRow;
+    if ((launches & 1) == 0) std::swap(pDest, pScratch);
+    for (unsigned left = numPasses; left;) {
+        const B26Shape shape = b26_shape(P.L, P.rows, P.iSpan, (int)left, wRow != 1);
+        left -= (unsigned)shape.passes;
+        P.passes = shape.passes;
+        P.lines = shape.lines;
+        P.wavesPerLine = shape.wavesPerLine;
+        P.haloWaves = shape.haloWaves;
+        P.blocks = (int)ckd_div_up(yRes, (unsigned)shape.lines);
+        P.colStride = left ? (int)xRes : (int)wCol;
+        P.rowStride = left ? 1 : (int)wRow;
+        switch (shape.per) {
+        case 3: launch_lines<3>(ctx, pDest, pRead, P); break;
+        case 5: launch_lines<5>(ctx, pDest, pRead, P); break;
+        case 7: launch_lines<7>(ctx, pDest, pRead, P); break;
+        default: launch_lines<9>(ctx, pDest, pRead, P); break;
         }
-        k_b26_pass<<<yRes, kBlock, lds, ctx->stream>>>(pDest, pRead, (int)xRes, (int)yRes, cs, rs, P);
         ckd_status s = ckd::check_launch("blur26 pass");
         if (s != CKD_OK) return s;
         pRead = pDest;
-        uint32_t *t = pDest;
-        pDest = pScratch;
-        pScratch = t;
+        std::swap(pDest, pScratch);
     }
     return CKD_OK;
 }

@@ -1,0 +1,69 @@
+"""The 2026 blur's line kernel (k_b26_lines) against the oracle, bit for bit:
+lines that fill their waves exactly, by one less and one more, for each number
+of pixels a lane takes; few lines and many, one and two a block; several passes a launch,
+where two pixels of the next line are carried along, up to as many as there are; spans from none to the longest; both store orders."""
+import numpy as np
+import pytest
+
+from helpers import rand_img
+from oracles import P
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ctx, orc, kind, W, H, strength, gain, passes):
+    print("blur26", kind, W, H, strength, gain, passes, flush=True)
+    n = W * H
+    src = np.zeros(n + 4, np.uint32)
+    src[:n] = rand_img(W + 3 * H, n)
+    want, s0, s1 = (np.zeros(n + 4, np.uint32) for _ in range(3))
+    {"h": orc.orc_blur26_h, "v": orc.orc_blur26_v, "2d": orc.orc_blur26}[kind](
+        P(want), P(src), W, H, strength, gain, passes, P(s0), P(s1))
+    d, s = ctx.empty(n), ctx.upload(src[:n])
+    {"h": ctx.blur26_h, "v": ctx.blur26_v, "2d": ctx.blur26}[kind](d, s, W, H, strength, gain, passes)
+    got = d.numpy()
+    assert np.array_equal(s.numpy(), src[:n])
+    ctx.free(s)
+    ctx.free(d)
+    bad = np.nonzero(got != want[:n])[0]
+    assert len(bad) == 0, (len(bad), int(bad[0]) // W, int(bad[0]) % W)
+
+
+WIDTHS = [4, 5, 191, 192, 193, 319, 320, 321, 448, 449, 576, 577, 639, 641, 960, 1080, 1151, 1152, 1153, 1344,
+          1728, 1919, 1920, 1921, 2047, 2048]
+
+
+@pytest.mark.parametrize("passes", [1, 2, 3, 7])
+@pytest.mark.parametrize("strength,gain", [(0.0, 0.0), (0.4, 1.0), (12.0, 0.0), (61.0, 0.5), (100.0, 1.0)])
+def test_line_lengths(ctx, orc, strength, gain, passes):
+    for W in WIDTHS:
+        _check(ctx, orc, "h", W, 5, strength, gain, passes)
+
+
+@pytest.mark.parametrize("passes", [1, 3, 4])
+@pytest.mark.parametrize("W,H", [(1920, 1027), (600, 2047), (321, 2048), (64, 1030)])
+def test_many_lines(ctx, orc, W, H, passes):
+    _check(ctx, orc, "h", W, H, 12.0, 0.0, passes)
+
+
+@pytest.mark.parametrize("passes", [1, 2, 3, 64])
+@pytest.mark.parametrize("kind,W,H", [("v", 1920, 1080), ("v", 1028, 516), ("2d", 2048, 320), ("2d", 4, 8)])
+def test_transposed_stores(ctx, orc, kind, W, H, passes):
+    _check(ctx, orc, kind, W, H, 3.0, 0.25, passes)
+
+
+@pytest.mark.parametrize("value", [0, 0xffffffff])
+def test_flat_images(ctx, orc, value):
+    """sums at their least and their greatest"""
+    W, H = 1925, 6
+    for strength, gain in [(0.0, 1.0), (0.2, 1.0), (100.0, 1.0), (100.0, 0.0)]:
+        n = W * H
+        src = np.full(n + 4, value, np.uint32)
+        src[n:] = 0
+        want, s0, s1 = (np.zeros(n + 4, np.uint32) for _ in range(3))
+        orc.orc_blur26_h(P(want), P(src), W, H, strength, gain, 3, P(s0), P(s1))
+        d, s = ctx.empty(n), ctx.upload(src[:n])
+        ctx.blur26_h(d, s, W, H, strength, gain, 3)
+        assert np.array_equal(d.numpy(), want[:n]), (strength, gain)
+        ctx.free(s)
+        ctx.free(d)
