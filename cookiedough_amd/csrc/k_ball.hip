@@ -357,20 +357,19 @@ __global__ __launch_bounds__(256) void k_ball(const BallJob *__restrict__ jobs, 
 // ---- Polar_BlitA ------------------------------------------------------------
 
 // Fetch16 through the map (code/polar.cpp:95-106), then the mix by the
-// fetched alpha: d + a*(s-d)/256 per channel (code/polar.cpp:157-174)
+// fetched alpha: d + a*(s-d)/256 per channel (code/polar.cpp:157-174).  Blocks of
+// 32x8 pixels and texels in pairs, as in k_polar_blit.
 __global__ __launch_bounds__(256) void k_polar_blit_a(uint32_t *__restrict__ dst,
                                                       const uint32_t *__restrict__ src,
                                                       const int2 *__restrict__ map, unsigned W,
                                                       unsigned H)
 {
-    const unsigned x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
+    const unsigned x = blockIdx.x * 32 + (threadIdx.x & 31), y = blockIdx.y * 8 + (threadIdx.x >> 5);
     if (x >= W || y >= H) return;
     const size_t i = (size_t)y * W + x;
     const int2 uv = map[i];
-    const unsigned U0 = (unsigned)(uv.x >> 8), V0 = (unsigned)(uv.y >> 8) * W;
-    const uint32_t s = ckd_bilerp32(src[U0 + V0], src[U0 + 1 + V0], src[U0 + V0 + W],
-                                    src[U0 + 1 + V0 + W], (uint32_t)uv.x & 0xff,
-                                    (uint32_t)uv.y & 0xff);
+    const uint32_t *p = src + (size_t)(uint32_t)(uv.y >> 8) * W + (uint32_t)(uv.x >> 8);
+    const uint32_t s = ckd_bilerp32(p[0], p[1], p[W], p[W + 1], (uint32_t)uv.x & 0xff, (uint32_t)uv.y & 0xff);
     const uint32_t a = s >> 24, d = dst[i];
     uint32_t r = 0;
 #pragma unroll
@@ -629,7 +628,7 @@ ckd_status ckd_polar_blit_a(ckd_ctx *ctx, uint32_t *dst, const uint32_t *src, un
     if (!pm)
         return ckd::fail(CKD_ESTATE, "ckd_polar_blit_a: no polar maps for %ux%u (ckd_polar_create)",
                          W, H);
-    dim3 grid(ckd_div_up(W, 256), H);
+    dim3 grid(ckd_div_up(W, 32), ckd_div_up(H, 8));
     k_polar_blit_a<<<grid, 256, 0, ctx->stream>>>(
         dst, src, reinterpret_cast<const int2 *>(inverse ? pm->inv : pm->map), W, H);
     return ckd::check_launch("polar_blit_a");
