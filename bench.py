@@ -281,7 +281,8 @@ def main() -> int:
                 "shades_evaluating_spheres": round(eval_shades / max(1, psdf["px"]), 4),
                 "algorithmic": "per launch: sum(steps)*18 + sphere_steps*88 + px*60 + "
                                "sphere_shades*528 FLOP: the spheres only where the bounding-sphere "
-                               "test did not rule them out"}
+                               "test did not rule them out (all 8 counted there, though a chunk may "
+                               "keep fewer)"}
     # HBM bytes per launch of this kernel on the 512-request batch, measured
     # with the FETCH_SIZE / WRITE_SIZE counters scaled by a copy of known size
     traffic = None
@@ -296,7 +297,8 @@ def main() -> int:
                 "launches": launches, "avg_launch_ms": round(ms_k / max(1, launches), 4),
                 "algorithmic": "per launch: sum(steps)*(F_sdf+7) + px*(6*F_sdf+40), "
                                "F_sdf = 11*8+2 = 90 FLOP (every sphere at every step, including those "
-                               "the bounding-sphere test skips exactly; `executed` counts only what runs)",
+                               "the bounding-sphere test and the chunks' lists skip exactly; `executed` "
+                               "leaves out the steps that evaluate none)",
                 "executed": executed}
     # the same kernel alone: the batch's SDF requests only, at their own
     # autotuned launch shape (in the batch it shares the GPU with the voxel
