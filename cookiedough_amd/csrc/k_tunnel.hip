@@ -339,6 +339,78 @@ __global__ __launch_bounds__(64) void k_tunnel_v(const TunJob *__restrict__ jobs
     for (; y < y1; ++y) edge_row(y);
 }
 
+// T2 for launches of few tiles (a single frame): a block of four waves takes the
+// 64 columns x kT2Seg rows that one wave of k_tunnel_v_ring walks down.  It reads
+// the tile's rows of tmp with e more either side into LDS, rows the image clips as
+// zeros, up to 16 rows a wave in flight; then each wave sums its first row's
+// window and slides it down a quarter of the rows.  A tile's time is its chain of
+// loads: 65 + 32 rows, eight at a time, in one wave against two rounds here.  A
+// frame of 1280x720, both passes: radius 32 32.5 -> 22.7 us, radius 33 (no ring)
+// 48.9 -> 22.4; 2560x1440 (1800 tiles) 59.2 -> 58.1 and 86.8 -> 58.3.  Many more
+// tiles fill the chip either way: 96 frames at 32-row segments 625 and 625 us, 200
+// of 640x360 296 and 324, so those stay with the ring, as do segments above 64 rows
+// (a quarter of them is a chain again) and windows that LDS does not hold.
+constexpr int kTileMaxSeg = 64, kTileMaxRows = 254; // of LDS: with D below 64 KiB
+constexpr unsigned kTileMaxTiles = 4096;
+__global__ __launch_bounds__(256) void k_tunnel_v_tile(const TunJob *__restrict__ jobs, int nJobs,
+                                                       const TunJob single, int kT2Seg)
+{
+    constexpr int U = 16, G = 8;
+    const uint32_t unit = blockIdx.x;
+    extern __shared__ uint32_t rows[]; // (kT2Seg + 2 * maxEdge) rows of 64 lanes
+    __shared__ __align__(16) uint16_t D[256];
+    const TunJob J = pick(jobs, nJobs, single, unit, &TunJob::vBase);
+    if (threadIdx.x < 64) copy_div_table<64>(D);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t local = unit - J.vBase;
+    const int x = (int)((local % J.vBlocksX) * 64) + lane;
+    const int y0 = (int)((local / J.vBlocksX) * kT2Seg);
+    const int W = (int)J.W, H = (int)J.H, e = (int)J.edge;
+    const int xc = min(x, W - 1);
+    const int y1 = min(y0 + kT2Seg, H), n = y1 - y0 + 2 * e;
+    const global_u32c *__restrict__ tmp = (const global_u32c *)J.tmp;
+    global_u32 *__restrict__ dst = (global_u32 *)J.dst;
+    uint32_t *mine = rows + lane; // row y0 - e + k in mine[64 * k]
+
+    const int per = (kT2Seg + 3) >> 2, ya = min(y0 + wave * per, y1), yb = min(ya + per, y1);
+    auto Drow = [&](int y) { return dst + (size_t)y * W; };
+    // rows past a group's last one read that row again, and are not used
+    uint32_t d[G];
+    auto load = [&](int y) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) d[j] = Drow(min(y + j, H - 1))[xc];
+    };
+    load(ya);
+    for (int k0 = wave * U; k0 < n; k0 += 4 * U) {
+        uint32_t v[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) v[j] = (tmp + (size_t)min(max(y0 - e + k0 + j, 0), H - 1) * W)[xc];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const int r = y0 - e + k0 + j;
+            if (k0 + j < n) mine[64 * (k0 + j)] = r >= 0 && r < H ? v[j] : 0u;
+        }
+    }
+    __syncthreads();
+    if (ya >= yb) return;
+    uint64_t F = 0;
+    const uint32_t *first = mine + 64 * (ya - y0);
+#pragma unroll 8
+    for (int k = 0; k <= 2 * e; ++k) F += ckd_spread(first[64 * k]);
+    for (int y = ya; y < yb; y += G) {
+        if (y != ya) load(y);
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+            const int yy = y + j;
+            if (yy >= yb) break;
+            const int lo = max(yy - e, 0), hi = min(yy + e, H - 1);
+            Drow(yy)[xc] = ckd_adds_u8x4(d[j], ckd_b07_div_pack(F, D[hi - lo + 1]));
+            const uint32_t *l = mine + 64 * (yy - y0);
+            if (yy + 1 < yb) F += ckd_spread(l[64 * (2 * e + 1)]) - ckd_spread(l[0]);
+        }
+    }
+}
+
 // T2 with the window in LDS: each wave keeps the 2e+1 rows of its 64
 // columns that the window spans, row r in slot r mod (2e+1), so the row
 // leaving the window comes from LDS instead of a second read of tmp (at
@@ -554,7 +626,12 @@ ckd_status launch_tunnel_jobs(ckd_ctx *ctx, const TunJob *jobs, int nJobs, const
     // the window ring holds up to 2 * kRingMaxEdge + 1 rows (16.6 KB per
     // wave); wider windows read their leaving rows again from memory
     const unsigned ringRows = tunnel_ring_rows(maxEdge);
-    if (ringRows)
+    const int seg = ctx->tuning.tunnelVSeg;
+    const int tileRows = seg + 2 * (int)maxEdge;
+    if (totalVBlocks <= kTileMaxTiles && seg <= kTileMaxSeg && tileRows <= kTileMaxRows)
+        k_tunnel_v_tile<<<totalVBlocks, 256, (size_t)tileRows * 64 * sizeof(uint32_t), ctx->stream>>>(jobs, nJobs, single,
+                                                                                                      seg);
+    else if (ringRows)
         k_tunnel_v_ring<8><<<totalVBlocks, 64, (size_t)ringRows * 64 * sizeof(uint32_t), ctx->stream>>>(
             jobs, nJobs, single, ctx->tuning.tunnelVSeg);
     else
