@@ -657,30 +657,36 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
 // bound (a square root and 8 more a sphere and step).  A 1280x720 frame with 8
 // spheres: 65 -> 39 us with the lists and the stretch.
 constexpr float kProbe = 1e-3f; // the normal's offset h
+constexpr int kFewSpheres = 6;
 
-template <bool kHalf>
+// kFew: few spheres in a frame of few tiles, where a ray's chain of steps is all
+// there is: every sphere on every step, from scalar registers.  cull: whether the
+// tile leaves spheres out (otherwise it keeps all).  Which is taken, and the times
+// either side of the lines: launch_sdf.
+template <bool kHalf, bool kFew>
 __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigned W, unsigned H, float invH,
-                                             const ckd_sdf_scene sc, const SdfCam cam, f4 bound,
+                                             const ckd_sdf_scene sc, const SdfCam cam, f4 bound, bool cull,
                                              unsigned long long *__restrict__ stepCount)
 {
     __shared__ f4 spheres[32]; // the tile's: centre, radius
     __shared__ uint32_t kept;  // their mask
     const unsigned lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned x0 = blockIdx.x * 16, y0 = blockIdx.y * 16;
-    if (wave == 0) {
+    if (!kFew && wave == 0) {
         const float c12[12] = {cam.o[0], cam.o[1], cam.o[2], cam.f[0], cam.f[1], cam.f[2],
                                cam.r[0], cam.r[1], cam.r[2], cam.u[0], cam.u[1], cam.u[2]};
         const uint32_t all = sc.nSpheres >= 32 ? 0xffffffffu : (1u << sc.nSpheres) - 1u;
-        const uint32_t keep = tile_spheres(sc, c12, bound, W, H, invH, x0, y0, min(16u, W - x0), min(16u, H - y0), lane,
-                                           all, 4.f * kProbe);
+        const uint32_t keep = cull ? tile_spheres(sc, c12, bound, W, H, invH, x0, y0, min(16u, W - x0),
+                                                  min(16u, H - y0), lane, all, 4.f * kProbe)
+                                   : all;
         if (lane < 32 && (keep >> lane & 1u))
             spheres[__popc(keep & ((1u << lane) - 1u))] =
                 f4{sc.sphere[lane][0], sc.sphere[lane][1], sc.sphere[lane][2], sc.sphere[lane][3]};
         if (lane == 0) kept = keep;
     }
-    __syncthreads();
-    const uint32_t keep = __builtin_amdgcn_readfirstlane(kept);
-    const int n = __popc(keep);
+    if (!kFew) __syncthreads();
+    const uint32_t keep = kFew ? (1u << sc.nSpheres) - 1u : __builtin_amdgcn_readfirstlane(kept);
+    const int n = kFew ? sc.nSpheres : __popc(keep);
     const unsigned x = x0 + (wave & 1) * 8 + (lane & 7), y = y0 + (wave >> 1) * 8 + (lane >> 3);
     int step = 0;
     if (x < W && y < H) {
@@ -694,12 +700,13 @@ __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigne
         dx *= il;
         dy *= il;
         dz *= il;
-        float tNear, tFar;
-        near_interval(cam.o[0] - bound.x, cam.o[1] - bound.y, cam.o[2] - bound.z, bound.w + 4.f * kProbe + origin_slack(cam.o),
+        float tNear = -INFINITY, tFar = INFINITY;
+        if (!kFew)
+            near_interval(cam.o[0] - bound.x, cam.o[1] - bound.y, cam.o[2] - bound.z, bound.w + 4.f * kProbe + origin_slack(cam.o),
                       cam.o[1] - sc.groundY, dx, dy, dz, 0.f, tNear, tFar);
         // distance of sphere i of the tile's from (px, py, pz)
         auto distance = [&](int i, float px, float py, float pz) {
-            const f4 c = spheres[i];
+            const f4 c = kFew ? f4{sc.sphere[i][0], sc.sphere[i][1], sc.sphere[i][2], sc.sphere[i][3]} : spheres[i];
             const float ex = px - c.x, ey = py - c.y, ez = pz - c.z;
             return fsqrt(fmaf(ez, ez, fmaf(ex, ex, ey * ey))) - c.w;
         };
@@ -710,8 +717,13 @@ __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigne
             hy = cam.o[1] + dy * total;
             hz = cam.o[2] + dz * total;
             d = hy - sc.groundY;
-            if (__ballot(total > tNear && total < tFar))
+            if (kFew) {
+#pragma unroll
+                for (int i = 0; i < kFewSpheres; ++i)
+                    if (i < n) d = fminf(d, distance(i, hx, hy, hz));
+            } else if (__ballot(total > tNear && total < tFar)) {
                 for (int i = 0; i < n; ++i) d = fminf(d, distance(i, hx, hy, hz));
+            }
             tHit = total;
             total += d;
         }
@@ -720,7 +732,7 @@ __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigne
         int id = sc.nSpheres;
         float p[6] = {hy - sc.groundY, hy - sc.groundY, hy + h - sc.groundY, hy - h - sc.groundY,
                       hy - sc.groundY, hy - sc.groundY};
-        if (__ballot(tHit > tNear && tHit < tFar)) {
+        if (kFew || __ballot(tHit > tNear && tHit < tFar)) {
             float best = hy - sc.groundY;
             uint32_t rest = keep;
             for (int i = 0; i < n; ++i) {
@@ -803,10 +815,24 @@ ckd_status launch_sdf(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigned H,
     const float invH = 1.0f / (float)H;
     const f4 bound = bounding_sphere(sc);
     KernelTimer kt(ctx, CKD_KT_SDF_PLAIN);
+    // Frames of few tiles wait for one ray's chain.  All spheres on every step, and
+    // tiles that keep all, against tiles that cull (us): 320x200 with 1 sphere 10.3
+    // / 14.5 / 15.1, 4: 20.6 / 27.1 / 26.7, 8: 34 / 28 / 45, 32: 119 / 84 / 77; 960x540
+    // with 4: 25.7 / 29.2 / 29.0, 8: 49 / 33 / 41, 16: 90 / 55 / 46; 1280x720 with 1:
+    // 17.1 / 18.5 / 19.1, 4: 33.1 / 31.6 / 30.3, 8: 68 / 41 / 42; 2560x1440 with 1: 54 /
+    // 46 / 50, 8: 189 / 87 / 70.
+    const uint64_t work = (uint64_t)grid.x * grid.y * (unsigned)sc.nSpheres;
+    const bool few = sc.nSpheres <= kFewSpheres && work < 10000, cull = work >= 24000 || sc.nSpheres > 16;
+    auto launch = [&](auto half, auto fewSpheres) {
+        k_sdf<decltype(half)::value, decltype(fewSpheres)::value>
+            <<<grid, 256, 0, ctx->stream>>>(dst, W, H, invH, sc, cam, bound, cull, stepCount);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
     if (shading == CKD_SHADE_FP16)
-        k_sdf<true><<<grid, 256, 0, ctx->stream>>>(dst, W, H, invH, sc, cam, bound, stepCount);
+        few ? launch(Yes{}, Yes{}) : launch(Yes{}, No{});
     else
-        k_sdf<false><<<grid, 256, 0, ctx->stream>>>(dst, W, H, invH, sc, cam, bound, stepCount);
+        few ? launch(No{}, Yes{}) : launch(No{}, No{});
     return check_launch("sdf");
 }
 

@@ -32,6 +32,15 @@ def test_sizes(ctx, orc, W, H, n):
     _check(ctx, orc, wl.sdf_scene(3, n, 64), W, H, 4.2)
 
 
+@pytest.mark.parametrize("W,H,n", [(640, 400, 6), (640, 400, 7), (800, 532, 6), (832, 536, 6), (640, 400, 16),
+                                   (640, 400, 17), (960, 540, 11), (960, 540, 12), (64, 64, 0)])
+def test_either_side_of_the_forms(ctx, orc, W, H, n):
+    """few spheres and few tiles; tiles that keep all spheres; tiles that cull"""
+    sc = wl.sdf_scene(3, max(n, 1), 64)
+    sc.nSpheres = n
+    _check(ctx, orc, sc, W, H, 4.2)
+
+
 @pytest.mark.parametrize("height", [-4.5, 0.0, 30.0])
 @pytest.mark.parametrize("radius", [0.5, 4.0, 40.0])
 def test_cameras_anywhere(ctx, orc, height, radius):
