@@ -420,10 +420,12 @@ ckd_status horz(ckd_ctx *ctx, uint32_t *pDest, uint32_t *pScratch, const uint32_
     P.halfScale = B.halfScale;
     P.dScale = B.dScale;
     // (sum * scale) >> 22 as the high half of a product of 24-bit factors with
-    // signs, 10 bits shared out between them: a sum is at most (2 iSpan + 2) * 255
-    // and a scale at most 2^22 / (iSpan + 1), so the two always fit
+    // signs, 10 bits shared out between them.  S0 - (T(0) + .. + T(iSpan)), what a
+    // sum holds beside its 2 iSpan + 1 terms of at most 255, is below 255 + iSpan +
+    // 1: rounding down takes less than 1 off each T.  A scale is at most 2^22 /
+    // (iSpan + 1), so the two always fit
     int sumBits = 0;
-    while (((2 * B.iSpan + 2) * 255) >> sumBits) ++sumBits;
+    while (((2 * B.iSpan + 2) * 255 + B.iSpan + 1) >> sumBits) ++sumBits;
     P.sumShift = std::min(10, 23 - sumBits);
     P.scaleShift = 10 - P.sumShift;
     P.scale = B.iScale << P.scaleShift;

@@ -67,3 +67,44 @@ def test_flat_images(ctx, orc, value):
         assert np.array_equal(d.numpy(), want[:n]), (strength, gain)
         ctx.free(s)
         ctx.free(d)
+
+
+def _span_strength(W, span, alpha):
+    """the strength whose radius on a line of W pixels is span + alpha"""
+    return 100.0 * (span + alpha) / ((W - 2) // 2)
+
+
+def _both_orders(ctx, orc, src, W, H, strength, gain, passes):
+    n = W * H
+    for kind in ("h", "v"):
+        w, h = (W, H) if kind == "h" else (H, W)
+        img = np.zeros(n + 4, np.uint32)
+        img[:n] = (src if kind == "h" else src.T).reshape(-1)
+        want, s0, s1 = (np.zeros(n + 4, np.uint32) for _ in range(3))
+        {"h": orc.orc_blur26_h, "v": orc.orc_blur26_v}[kind](
+            P(want), P(img), w, h, strength, gain, passes, P(s0), P(s1))
+        d, s = ctx.empty(n), ctx.upload(img[:n])
+        {"h": ctx.blur26_h, "v": ctx.blur26_v}[kind](d, s, w, h, strength, gain, passes)
+        got = d.numpy()
+        ctx.free(s)
+        ctx.free(d)
+        bad = np.nonzero(got != want[:n])[0]
+        assert len(bad) == 0, (kind, len(bad), int(bad[0]) // w, int(bad[0]) % w)
+
+
+@pytest.mark.parametrize("gain", [0.0, 1.0])
+@pytest.mark.parametrize("span", [1, 3, 15, 63, 127, 255, 256, 257, 500])
+def test_sums_above_the_flat_image(ctx, orc, span, gain):
+    """the terms subtracted are rounded down, so a line that is random where
+    they come from and 255 elsewhere has sums above the flat image's: at a span
+    of 256 they pass 2^17"""
+    W, H = 1024, 8
+    rng = np.random.default_rng(span)
+    line = np.full((H, W, 4), 255, np.uint8)
+    line[:, 1:span] = rng.integers(0, 256, (H, span - 1, 4))
+    line[:, span:span + 2] = 0
+    src = np.ascontiguousarray(line).view(np.uint32).reshape(H, W)
+    strength = _span_strength(W, span, 0.997) if span < 500 else 100.0
+    for passes in (1, 2):
+        print("sums", span, gain, passes, flush=True)
+        _both_orders(ctx, orc, src, W, H, strength, gain, passes)
