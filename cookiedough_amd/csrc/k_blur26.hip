@@ -180,9 +180,12 @@ void k_b26_lines(uint32_t *__restrict__ out, const uint32_t *__restrict__ in, co
     const int base = w * 64 * kPer, j0 = base + lane * kPer; // the lane's first pixel
     Pairs *T = lds + slot * stride + iSpan + 1;              // T[0]: of pixel 0
 
+    // zeros either side; the halo's from its last wave on: a lane with its last
+    // needed pixels may hold others that read past it, and the lane's sums keep to
+    // 16 bits only if all its terms do
+    const int held = slotWaves * 64 * kPer; // pixels of the slot's waves
     for (int i = w * 64 + lane; i <= iSpan; i += slotWaves * 64) T[i - iSpan - 1] = {0, 0};
-    if (!halo)
-        for (int i = L + 1 + w * 64 + lane; i <= reach + iSpan; i += slotWaves * 64) T[i] = {0, 0};
+    for (int i = (halo ? held : L + 1) + w * 64 + lane; i <= held + iSpan; i += slotWaves * 64) T[i] = {0, 0};
     if (base > iSpan && lane < 4) starts[4 * wave + lane] = 0;
 
     // the line's pixels, and the two after it (last wave)

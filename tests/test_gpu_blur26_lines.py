@@ -74,7 +74,7 @@ def _span_strength(W, span, alpha):
     return 100.0 * (span + alpha) / ((W - 2) // 2)
 
 
-def _both_orders(ctx, orc, src, W, H, strength, gain, passes):
+def _both_orders(ctx, orc, src, W, H, strength, gain, passes, before=lambda: None):
     n = W * H
     for kind in ("h", "v"):
         w, h = (W, H) if kind == "h" else (H, W)
@@ -84,6 +84,7 @@ def _both_orders(ctx, orc, src, W, H, strength, gain, passes):
         {"h": orc.orc_blur26_h, "v": orc.orc_blur26_v}[kind](
             P(want), P(img), w, h, strength, gain, passes, P(s0), P(s1))
         d, s = ctx.empty(n), ctx.upload(img[:n])
+        before()
         {"h": ctx.blur26_h, "v": ctx.blur26_v}[kind](d, s, w, h, strength, gain, passes)
         got = d.numpy()
         ctx.free(s)
@@ -108,3 +109,26 @@ def test_sums_above_the_flat_image(ctx, orc, span, gain):
     for passes in (1, 2):
         print("sums", span, gain, passes, flush=True)
         _both_orders(ctx, orc, src, W, H, strength, gain, passes)
+
+
+# two or three passes of a launch whose halo waves hold barely the pixels
+# needed, for 3, 5, 7 and 9 pixels a lane
+@pytest.mark.parametrize("W,H,span,passes", [
+    (1024, 40, 189, 2), (1024, 40, 190, 2), (1024, 40, 382, 2), (1024, 300, 190, 2), (1024, 40, 191, 2),
+    (1920, 1032, 315, 2), (1920, 1032, 317, 2), (1920, 1032, 318, 2), (1344, 1032, 443, 2), (1344, 1032, 446, 2),
+    (1024, 40, 94, 3), (1920, 1032, 158, 3), (1600, 1032, 284, 3), (1600, 1032, 286, 3)])
+def test_halo_of_the_next_line(ctx, orc, W, H, span, passes):
+    """every launch after one of another kernel that leaves pixels in LDS"""
+    rng = np.random.default_rng(W + span)
+    noise = rng.integers(0, 1 << 32, (H, W), dtype=np.uint64).astype(np.uint32)
+    dark = noise & np.uint32(0x1f1f1f1f)
+    lines = rng.integers(0, 1 << 32, (2048, 2000), dtype=np.uint64).astype(np.uint32).reshape(-1)
+    t = ctx.upload(lines)
+
+    def leave_pixels():
+        ctx.blur07_inplace_batch([t], [7.5 / 255.0], 2000, 2048, 1)
+
+    print("halo", W, H, span, passes, flush=True)
+    for src in (noise, dark):
+        _both_orders(ctx, orc, src, W, H, _span_strength(W, span, 0.4), 0.0, passes, leave_pixels)
+    ctx.free(t)
