@@ -28,7 +28,7 @@ ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, ui
 void tunnel_job_geometry(TunJob &J, uint32_t *dst, uint32_t *tmp, const int32_t *grid, unsigned W,
                          unsigned H, int radius);
 uint32_t tunnel_vblocks(unsigned W, unsigned H, int seg);
-unsigned tunnel_ring_rows(unsigned maxEdge);
+unsigned tunnel_captured_edge(unsigned maxEdge);
 ckd_status launch_tunnel_jobs(ckd_ctx *ctx, const TunJob *jobs, int nJobs, const TunJob &single,
                               uint32_t totalRows, uint32_t totalVBlocks, unsigned maxW,
                               unsigned maxEdge, const uint32_t *tex, uint4 *quads, unsigned texLog2,
@@ -57,9 +57,8 @@ struct ckd_graph {
     size_t tmpPixels = 0;
     int nSpheres = 0;
     std::vector<ReqShape> shapes;
-    // window rows of the captured vertical-blur ring (0: no ring): the
-    // largest radius a replay can take
-    unsigned tunRingRows = 0;
+    // the largest tunnel radius that a replay can take (tunnel_captured_edge)
+    unsigned tunMaxE = 0;
     uint4 *quads = nullptr;
 };
 
@@ -404,7 +403,7 @@ ckd_status ckd_batch_graph_create(ckd_ctx *ctx, const ckd_request *requests, uns
     g->tmp = tmp;
     g->nSpheres = scene ? scene->nSpheres : 0;
     g->tmpPixels = tmpPixels;
-    g->tunRingRows = P.nTun ? ckd::tunnel_ring_rows(P.tunMaxE) : 0;
+    P.tunMaxE = g->tunMaxE = ckd::tunnel_captured_edge(P.tunMaxE);
     for (unsigned i = 0; i < n; ++i)
         g->shapes.push_back({requests[i].effect, requests[i].W, requests[i].H});
     if (ckd::dev_alloc(&g->tables, P.host.size()) != hipSuccess) {
@@ -485,10 +484,10 @@ ckd_status ckd_graph_update(ckd_graph *g, const ckd_request *requests, unsigned 
     make_plan(g->tuning, requests, n, g->tmp, g->nSpheres, P);
     if (P.host.size() != g->tableBytes)
         return ckd::fail(CKD_EINVAL, "ckd_graph_update: the requests' tables do not fit the graph");
-    if (g->tunRingRows && 2 * P.tunMaxE + 1 > g->tunRingRows)
+    if (P.tunMaxE > g->tunMaxE)
         return ckd::fail(CKD_EINVAL,
                          "ckd_graph_update: radius %u exceeds the captured batch's largest (%u)",
-                         P.tunMaxE, (g->tunRingRows - 1) / 2);
+                         P.tunMaxE, g->tunMaxE);
     // a replay still in flight reads the tables: the copy waits for it, and
     // the next replay is queued after the copy
     ckd_ctx *ctx = g->ctx;

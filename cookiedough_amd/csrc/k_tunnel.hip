@@ -350,7 +350,8 @@ __global__ __launch_bounds__(64) void k_tunnel_v(const TunJob *__restrict__ jobs
 // tiles fill the chip either way: 96 frames at 32-row segments 625 and 625 us, 200
 // of 640x360 296 and 324, so those stay with the ring, as do segments above 64 rows
 // (a quarter of them is a chain again) and windows that LDS does not hold.
-constexpr int kTileMaxSeg = 64, kTileMaxRows = 254; // of LDS: with D below 64 KiB
+constexpr int kTileMaxSeg = 64, kTileMaxRows = 254; // of LDS: with D 64 KiB
+static_assert(8 + 2 * 127 > kTileMaxRows, "no tile holds the widest window (tunnel_captured_edge)");
 constexpr unsigned kTileMaxTiles = 4096;
 __global__ __launch_bounds__(256) void k_tunnel_v_tile(const TunJob *__restrict__ jobs, int nJobs,
                                                        const TunJob single, int kT2Seg)
@@ -592,6 +593,12 @@ unsigned tunnel_ring_rows(unsigned maxEdge)
 {
     return maxEdge <= (unsigned)kRingMaxEdge ? 2 * maxEdge + 1 : 0;
 }
+
+// The largest window edge that a captured launch has to be able to take, which
+// is what launch_tunnel_jobs is then given: a graph's radii change with its job
+// tables, but not its kernel and its LDS.  Up to the ring's limit updates keep
+// to the captured edge; past it they may bring any, which only k_tunnel_v takes.
+unsigned tunnel_captured_edge(unsigned maxEdge) { return maxEdge <= (unsigned)kRingMaxEdge ? maxEdge : 127; }
 
 size_t tex_quad_bytes(unsigned texLog2)
 {
