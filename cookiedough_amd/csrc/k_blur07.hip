@@ -22,6 +22,7 @@
 #include "ckd_internal.h"
 #include "ckd_pixel.h"
 #include "ckd_b07.h"
+#include "ckd_b07_scan.h"
 
 #include <vector>
 
@@ -758,7 +759,7 @@ CKD_DEV void b07_scan_line(uint8_t *px, int len, const B07Params &p, const uint1
     for (; p0 <= em && p0 < nSteps; p0 += kSteps) edge_chunk(p0);
     // whole chunks inside the middle run: back > 0, pos < len - 1 and pos <
     // nSteps, full divisor; the next chunk's pixels are read ahead
-    const int last = len - 1 - 16;
+    const int last = ckd::b07_scan_last(len, nSteps);
     if (p0 <= last) {
         const uint8_t *in = px + 4 * (p0 + t), *from = in - 4 * em;
         uint8_t *to = px + 4 * (p0 + t - e);
