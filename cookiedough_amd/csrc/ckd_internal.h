@@ -79,6 +79,7 @@ struct ckd_ctx {
     uint32_t lsFog0 = 0;
     uint32_t *lsQuadH = nullptr;
     uint4 *lsQuadC = nullptr;
+    bool lsReady = false; // the last ckd_landscape_create succeeded
     // the fog table in 16-bit lanes and the span lengths' divisors
     uint2 *lsFogLanes = nullptr;
     uint16_t *lsSpanDiv = nullptr;

@@ -660,7 +660,7 @@ ckd_status launch_landscape_jobs(ckd_ctx *ctx, const VoxJob *jobs, int nJobs, ui
                                  unsigned blockCols)
 {
     if (totalBlocks == 0) return CKD_OK;
-    if (!ctx->lsHeight)
+    if (!ctx->lsReady)
         return fail(CKD_ESTATE, "voxel requests need the landscape maps (ckd_landscape_create)");
     KernelTimer kt(ctx, CKD_KT_LANDSCAPE);
     const LsMaps M = ls_maps(ctx);
@@ -684,6 +684,7 @@ ckd_status ckd_landscape_create(ckd_ctx *ctx, const uint8_t *heightMap, const ui
     CKD_REQUIRE(heightMap && colorMap && fog256, "ckd_landscape_create: null map");
     CKD_REQUIRE_CTX(ctx);
     CKD_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->lsReady = false; // until every table below is whole
     ckd_status s = upload(heightMap, 1024 * 1024, (void **)&ctx->lsHeight);
     if (s == CKD_OK) s = upload(colorMap, 1024 * 1024 * 4, (void **)&ctx->lsColor);
     if (s == CKD_OK) s = upload(fog256, 256 * 4, (void **)&ctx->lsFog);
@@ -700,8 +701,10 @@ ckd_status ckd_landscape_create(ckd_ctx *ctx, const uint8_t *heightMap, const ui
     k_ls_quads<<<kTexels / 256, 256, 0, ctx->stream>>>(ctx->lsHeight, ctx->lsColor, ctx->lsQuadH,
                                                        ctx->lsQuadC);
     s = ckd::check_launch("landscape quads and tables");
-    if (s == CKD_OK) CKD_HIP(hipStreamSynchronize(ctx->stream));
-    return s;
+    if (s != CKD_OK) return s;
+    CKD_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->lsReady = true;
+    return CKD_OK;
 }
 
 ckd_status ckd_landscape_draw(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigned H,
@@ -716,7 +719,7 @@ ckd_status ckd_landscape_draw(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigned 
         CKD_REQUIRE(cams[f].mapTilt >= 0 && cams[f].mapTilt <= 180,
                     "ckd_landscape_draw: frame %u: mapTilt %d outside 0..180", f, cams[f].mapTilt);
     CKD_REQUIRE_CTX(ctx);
-    if (!ctx->lsHeight) return ckd::fail(CKD_ESTATE, "ckd_landscape_draw: no maps (ckd_landscape_create)");
+    if (!ctx->lsReady) return ckd::fail(CKD_ESTATE, "ckd_landscape_draw: no maps (ckd_landscape_create)");
     LsLaunch P;
     memset(&P, 0, sizeof(P));
     P.rayY = ls_rayY(W, H);

@@ -11,7 +11,7 @@ import pytest
 
 from cookiedough_amd import _lib
 from cookiedough_amd import workloads as wl
-from cookiedough_amd._lib import CKD_ENOMEM, CkdError
+from cookiedough_amd._lib import CKD_ENOMEM, CKD_ESTATE, CkdError
 from cookiedough_amd.device import Context
 from helpers import rand_img
 
@@ -130,3 +130,45 @@ def test_lazy_scratch_paths_recover(lib):
                 results.append(o.numpy())
                 g.close()
         assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
+
+
+def _refused(fn):
+    with pytest.raises(CkdError) as ei:
+        fn()
+    assert ei.value.status == CKD_ESTATE, str(ei.value)
+
+
+def test_landscape_after_a_failed_create(lib):
+    """whichever allocation of a create fails, the first one or a later one, the
+    context has no landscape to draw, alone or in a batch, until one succeeds"""
+    W, H = 320, 180
+    m, path = wl.landscape_maps(0), wl.landscape_path(0)
+    cam = wl.landscape_cam(path, 0.3)
+    with Context(0) as c:
+        d = c.empty(W * H)
+        req = c.request_array([wl.make_request(wl.BatchItem(1, W, H, 2.0), d.ptr, None, path, None)])
+
+        def create():
+            c.landscape_create(m.height, m.color, m.fog)
+
+        def refused():
+            _refused(lambda: c.landscape_draw(d, W, H, [cam]))
+            _refused(lambda: c.render_batch(req, None, 1, None, 9, None, 0))
+
+        refused()
+        for n in range(6):
+            lib.ckd_debug_fail_alloc(n)
+            _expect_enomem(create)
+            refused()
+        create()
+        c.landscape_draw(d, W, H, [cam])
+        c.sync()
+        first = d.numpy()
+        for n in range(3):
+            lib.ckd_debug_fail_alloc(n)
+            _expect_enomem(create)
+            refused()
+        create()
+        c.landscape_draw(d, W, H, [cam])
+        c.sync()
+        assert np.array_equal(d.numpy(), first)
