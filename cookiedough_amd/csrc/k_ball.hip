@@ -702,6 +702,7 @@ ckd_status ckd_twister_create(ckd_ctx *ctx, const uint8_t *heightMap, const uint
     if (ctx->twBackground && (ctx->twW != W || ctx->twH != H)) {
         CKD_HIP(hipFree(ctx->twBackground));
         ctx->twBackground = nullptr;
+        ctx->twW = ctx->twH = 0; // nothing to draw if the new one fails
     }
     if (!ctx->twBackground && ckd::dev_alloc(&ctx->twBackground, (size_t)W * H * 4) != hipSuccess)
         return ckd::fail(CKD_ENOMEM, "ckd_twister_create: cannot allocate the background");
@@ -809,6 +810,7 @@ ckd_status ckd_ball_create(ckd_ctx *ctx, const uint8_t *heightMaps5, const uint3
     if (ctx->ballImages && (ctx->ballW != W || ctx->ballH != H)) {
         CKD_HIP(hipFree(ctx->ballImages));
         ctx->ballImages = nullptr;
+        ctx->ballW = ctx->ballH = 0; // nothing to draw if the new ones fail
     }
     // two backgrounds and the halo, then the fan deltas of the H rays
     const size_t fanOffset = ((size_t)3 * W * H * 4 + 255) & ~(size_t)255;

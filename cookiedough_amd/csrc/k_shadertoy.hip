@@ -1250,7 +1250,7 @@ ckd_status ckd_fdtunnel_map(ckd_ctx *ctx, uint32_t *maps, uint32_t *glowMaps, un
     if (s != CKD_OK || (s = check_params("ckd_fdtunnel_map", frames, nFrames)) != CKD_OK) return s;
     CKD_REQUIRE(glowMaps, "ckd_fdtunnel_map: null glow maps");
     CKD_REQUIRE_CTX(ctx);
-    CKD_REQUIRE(ctx->fdTex, "ckd_fdtunnel_map: no textures (ckd_fdtunnel_create)");
+    CKD_REQUIRE(ctx->fdTex && ctx->fdTexHi, "ckd_fdtunnel_map: no textures (ckd_fdtunnel_create)");
     return st_maps(ctx, FX_FDTUNNEL, frames, nFrames, maps, glowMaps, resX, resY, false);
 }
 
@@ -1260,7 +1260,7 @@ ckd_status ckd_fdtunnel_draw(ckd_ctx *ctx, uint32_t *dst, unsigned resX, unsigne
     ckd_status s = check_geometry("ckd_fdtunnel_draw", resX, resY, nFrames, dst, frames);
     if (s != CKD_OK || (s = check_params("ckd_fdtunnel_draw", frames, nFrames)) != CKD_OK) return s;
     CKD_REQUIRE_CTX(ctx);
-    CKD_REQUIRE(ctx->fdTex, "ckd_fdtunnel_draw: no textures (ckd_fdtunnel_create)");
+    CKD_REQUIRE(ctx->fdTex && ctx->fdTexHi, "ckd_fdtunnel_draw: no textures (ckd_fdtunnel_create)");
     return st_draw(ctx, FX_FDTUNNEL, frames, nFrames, dst, resX, resY, false);
 }
 

@@ -773,7 +773,7 @@ ckd_status ckd_tunnelscape_rows(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigne
     CKD_REQUIRE(W >= 8 && H >= 8 && W <= 4096 && H <= 4096, "ckd_tunnelscape_rows: bad size %ux%u",
                 W, H);
     CKD_REQUIRE_CTX(ctx);
-    if (!ctx->tsHeight)
+    if (!ctx->tsHeight || !ctx->tsColor || !ctx->tsFog)
         return ckd::fail(CKD_ESTATE, "ckd_tunnelscape_rows: no maps (ckd_tunnelscape_create)");
     // tscape (code/tunnelscape.cpp:103-118) frame constants, host FP32
     float mapStepX, fromXAdd;

@@ -172,3 +172,58 @@ def test_landscape_after_a_failed_create(lib):
         c.landscape_draw(d, W, H, [cam])
         c.sync()
         assert np.array_equal(d.numpy(), first)
+
+
+def test_other_maps_after_a_failed_create(lib):
+    """the same for the tunnelscape's maps, the tunnel's textures, and the ball
+    and the twister, whose images are allocated again for another size"""
+    W, H = 1280, 64
+
+    def fails(create, allocs, draw):
+        for n in range(allocs):
+            lib.ckd_debug_fail_alloc(n)
+            _expect_enomem(create)
+            with pytest.raises(CkdError):
+                draw()
+        create()
+        draw()
+
+    m = wl.tunnelscape_maps(0)
+    tex = rand_img(5, 1 << 20)
+    tw = _lib.TwisterParams(time=1.0, **dict(wl.TWISTER_DEMO, blur=0.0))
+    ball = _lib.BallParams(time=1.0, **dict(wl.BALL_DEMO[1], radius=100.0))
+    fd = _lib.ST_PARAMS["fdtunnel"](time=1.0, **wl.ST_DEMO["fdtunnel"])
+    with Context(0) as c:
+        d, t = c.empty(W * H), c.empty(2 * W * H)
+
+        def tunnelscape():
+            c.tunnelscape_create(m.height, m.color, m.fog)
+
+        fails(tunnelscape, 3, lambda: c.tunnelscape_rows(d, W, H, 0.14, 0.6, 40.0, 1.0))
+        fails(tunnelscape, 3, lambda: c.tunnelscape_rows(d, W, H, 0.14, 0.6, 40.0, 1.0))
+        # an allocation that succeeded stays: the second create starts at the other
+        fails(lambda: c.fdtunnel_create(tex, tex), 2, lambda: c.st_draw("fdtunnel", d, W, H, [fd]))
+        for kind, maps, prm in (("twister", wl.twister_maps, tw), ("ball", wl.ball_maps, ball)):
+            def create(w, h):
+                mm = maps(w, h)
+                if kind == "ball":
+                    c.ball_create(mm, w, h)
+                else:
+                    c.twister_create(mm["heightMap"], mm["colorMap"], mm["background"], w, h)
+
+            def draw(w, h):
+                getattr(c, kind + "_draw")(d, t, w, h, [prm])
+
+            create(W, H)
+            draw(W, H)
+            c.polar_create(W, H // 2)
+            lib.ckd_debug_fail_alloc(0)
+            _expect_enomem(lambda: create(W, H // 2))
+            with pytest.raises(CkdError):
+                draw(W, H // 2)
+            # the old size's images went with it
+            with pytest.raises(CkdError):
+                draw(W, H)
+            create(W, H // 2)
+            draw(W, H // 2)
+            c.sync()
