@@ -980,30 +980,43 @@ int ring_k(unsigned mLo) { return mLo >= 8 ? 8 : mLo >= 4 ? 4 : mLo >= 2 ? 2 : 1
 // smallest median of the batch allows (0: none); its lines per block (their LDS
 // within 64 KiB) and its grid.  One wave takes a line, so its time grows with
 // the lines per SIMD and with the chunks of a line, where the kernels above
-// take one line's time until they have filled the chip: it is taken up to (steps
-// - 2) * 5 / 4 lines per SIMD.  Measured at 1280x720, rows and columns, us,
-// scan against the better of the others: span 82 (16 steps) 1 frame 21 and 18
-// against 74 and 71, 8 frames 48 and 50 against 75 and 88, 16 frames 85 and 83
-// against 151 and 90, 48 frames 218 and 223 against 206 and 146; span 22 (10
-// steps) 8 frames 71 and 70 against 75 and 86, 16 frames 131 and 122 against
-// 148 and 88; span 10 (4 steps) 8 frames 113 and 104 against 80 and 86.
+// take one line's time until they have filled the chip.  It is taken up to (steps
+// - 2) * 5 / 4 lines per SIMD, and
+// - fewer where lines are short and their chunks nearly all edges: along the rows
+//   below 640 pixels (1024 with fewer steps), along the columns below 128;
+// - along columns too long for a block of four (rows of 4- and 8-byte pieces then)
+//   only as many as about a third of the steps in rounds of resident blocks.
+// Measured at 1280x720, rows and columns, us, scan against the better of the
+// others: span 82 (16 steps) 1 frame 21 and 18 against 74 and 71, 8 frames 48 and
+// 50 against 75 and 88, 16 frames 85 and 83 against 151 and 90, 48 frames 218 and
+// 223 against 206 and 146; span 22 (10 steps) 8 frames 71 and 70 against 75 and
+// 86, 16 frames 131 and 122 against 148 and 88; span 10 (4 steps) 8 frames 113 and
+// 104 against 80 and 86.  Scan's share of their time, 16 steps, along rows of 64
+// pixels 0.94 with 6144 lines, 1.36 with 12288; of 512, 0.71 with 8192, 1.13 with
+// 16000; along columns of 4096 pixels 0.90 with 8192, 1.10 with 16000; of 16000, 0.57
+// with 2048, 1.21 with 4096; at 4 steps 0.85 with 1024 and 1.65 with 2048.
 struct ScanShape {
     int steps = 0, lines = 0;
     unsigned blocks = 0;
     size_t lds = 0;
     dim3 grid(unsigned n) const { return dim3((blocks + 7) / 8 * 8, n); }
 };
-ScanShape scan_shape(const ckd_ctx *ctx, unsigned mLo, int nLines, int len, unsigned n)
+ScanShape scan_shape(const ckd_ctx *ctx, unsigned mLo, int nLines, int len, bool columns, unsigned n)
 {
     ScanShape S;
-    const size_t line = (size_t)(len + kScanPad) * 4;
+    const size_t line = (size_t)(len + kScanPad) * 4, cus = (size_t)ctx->cuCount;
     if (mLo < 4 || line > 65536) return S;
     const int steps = mLo >= 16 ? 16 : mLo >= 12 ? 12 : mLo >= 10 ? 10 : mLo >= 8 ? 8 : mLo >= 6 ? 6 : 4;
-    if ((size_t)nLines * n * 4 > (size_t)(steps - 2) * 5 * 4 * (size_t)ctx->cuCount) return S;
-    S.steps = steps;
+    const size_t all = (size_t)nLines * n;
+    size_t most = (size_t)(steps - 2) * 5 * cus;
+    if (len < (columns ? 128 : steps < 16 ? 1024 : 640)) most = most * len / (len + (columns ? 6 : 12) * (steps - 4));
+    if (all > most) return S;
     S.lines = kScanLines;
     while ((size_t)S.lines * line > 65536) S.lines >>= 1;
     S.lds = (size_t)S.lines * line;
+    const size_t resident = 160 * 1024 / (S.lds + 512) * S.lines * cus; // with the divisors' 512 bytes
+    if (columns && S.lines < kScanLines && all * 25 > resident * (size_t)(8 * steps + 3)) return S;
+    S.steps = steps;
     S.blocks = ckd_div_up((size_t)nLines, (size_t)S.lines);
     return S;
 }
@@ -1012,7 +1025,7 @@ ckd_status launch_inplace(ckd_ctx *ctx, uint32_t *img, int nLines, int len, size
                           size_t pixStride, const B07Params &p, const char *what)
 {
     const int nl = lines_per_block(len);
-    if (const ScanShape S = scan_shape(ctx, p.median, nLines, len, 1); S.steps) {
+    if (const ScanShape S = scan_shape(ctx, p.median, nLines, len, pixStride != 1, 1); S.steps) {
         B07Job job;
         job.img = img;
         job.p = p;
@@ -1147,7 +1160,7 @@ ckd_status blur07_inplace_jobs(ckd_ctx *ctx, const B07Job *hostJobs, const B07Jo
         ring = columns || blocks > perCU * (size_t)ctx->cuCount;
     }
     const char *what = columns ? "blur07_v (in place, batch)" : "blur07_h (in place, batch)";
-    const ScanShape S = ctx->tuning.blurKernel == 0 ? scan_shape(ctx, mLo, (int)nLines, (int)len, n) : ScanShape();
+    const ScanShape S = ctx->tuning.blurKernel == 0 ? scan_shape(ctx, mLo, (int)nLines, (int)len, columns, n) : ScanShape();
     if (S.steps) {
         const int cols = columns ? 1 : 0, threads = S.lines * 64;
         switch (S.steps) {

@@ -60,11 +60,23 @@ def test_longest_lines(ctx, orc, length, lines, passes):
     _check(ctx, orc, W, H, 1, [76], passes, "noise", 7)
 
 
-# 256 CUs: 2560 lines at 4 steps a chunk, 17920 at 16
+# 256 CUs: 2560 lines at 4 steps a chunk; 17920 lines of 96 pixels are past the
+# limit at 16 (test_limits_by_length)
 @pytest.mark.gpu
 @pytest.mark.parametrize("span,lines,n", [(8, 1280, 2), (8, 1281, 2), (40, 1280, 14), (40, 1281, 14)])
 def test_batch_limit(ctx, orc, span, lines, n):
     _check(ctx, orc, 96, lines, n, [span, span + 3], 1, "runs", 90)
+
+
+# 256 CUs again, where the scan gives way sooner: rows of 96 pixels at 16 steps
+# from 7168 lines on, columns of 96 at 10 steps from 7447, columns of 16000
+# pixels, two blocks of one a CU, from 716 at 4 steps
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,H,n,span,passes", [
+    (96, 1024, 7, 40, 1), (96, 1025, 7, 40, 1), (1063, 96, 7, 22, 2), (1064, 96, 7, 22, 2),
+    (716, 16000, 1, 10, 2), (717, 16000, 1, 10, 2)])
+def test_limits_by_length(ctx, orc, W, H, n, span, passes):
+    _check(ctx, orc, W, H, n, [span, span + 3], passes, "noise", 91)
 
 
 def test_clamped_additions_compose():
