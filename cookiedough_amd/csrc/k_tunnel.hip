@@ -345,14 +345,19 @@ __global__ __launch_bounds__(64) void k_tunnel_v(const TunJob *__restrict__ jobs
 // zeros, up to 16 rows a wave in flight; then each wave sums its first row's
 // window and slides it down a quarter of the rows.  A tile's time is its chain of
 // loads: 65 + 32 rows, eight at a time, in one wave against two rounds here.  A
-// frame of 1280x720, both passes: radius 32 32.5 -> 22.7 us, radius 33 (no ring)
-// 48.9 -> 22.4; 2560x1440 (1800 tiles) 59.2 -> 58.1 and 86.8 -> 58.3.  Many more
-// tiles fill the chip either way: 96 frames at 32-row segments 625 and 625 us, 200
-// of 640x360 296 and 324, so those stay with the ring, as do segments above 64 rows
-// (a quarter of them is a chain again) and windows that LDS does not hold.
+// frame of 1280x720, both passes: radius 12 20.3 -> 15.8 us, 32 27.7 -> 17.6, 33 (no
+// ring) 43.8 -> 17.6, 64 58.2 -> 19.8, 111 69.8 -> 23.0; 2560x1440 (1800 tiles) radius 12
+// 34.1 -> 29.9, 33 64.5 -> 35.2, 111 94.8 -> 60.6.  Many more tiles fill the chip either
+// way: 96 frames at 32-row segments 625 and 625 us, 200 of 640x360 296 and 324, so
+// those stay with the ring, as do segments above 64 rows (a quarter of them is a chain
+// again) and windows that LDS does not hold.  Short segments read the window's rows
+// again for few of their own: at 8 rows 1400 tiles (1280x560, radius 12) 17.6 -> 15.9 us,
+// but 2825 (1600x900) 23.3 -> 24.8 at radius 16 and 4050 (1920x1080) 25.4 -> 30.4 at
+// radius 6; at 16 rows 2040 24.2 -> 26.0 at radius 6, 27.7 -> 27.5 at 12.  Past the ring
+// they win up to 4050 tiles of 198 rows (79 -> 68 us) and lose at 214 (81.7 -> 87.2).
 constexpr int kTileMaxSeg = 64, kTileMaxRows = 254; // of LDS: with D 64 KiB
 static_assert(8 + 2 * 127 > kTileMaxRows, "no tile holds the widest window (tunnel_captured_edge)");
-constexpr unsigned kTileMaxTiles = 4096;
+constexpr unsigned kTileMaxTiles = 4096, kTileMaxShort = 1500, kTileMaxReads = 860000;
 __global__ __launch_bounds__(256) void k_tunnel_v_tile(const TunJob *__restrict__ jobs, int nJobs,
                                                        const TunJob single, int kT2Seg)
 {
@@ -635,7 +640,11 @@ ckd_status launch_tunnel_jobs(ckd_ctx *ctx, const TunJob *jobs, int nJobs, const
     const unsigned ringRows = tunnel_ring_rows(maxEdge);
     const int seg = ctx->tuning.tunnelVSeg;
     const int tileRows = seg + 2 * (int)maxEdge;
-    if (totalVBlocks <= kTileMaxTiles && seg <= kTileMaxSeg && tileRows <= kTileMaxRows)
+    // many tiles of short segments read their windows' rows too often: kept for the
+    // wider windows of 16 to 23 rows and for windows the ring does not hold
+    const bool shortTiles = totalVBlocks > kTileMaxShort && seg < 24 && (seg < 16 || maxEdge < 8);
+    if (totalVBlocks <= kTileMaxTiles && seg <= kTileMaxSeg && tileRows <= kTileMaxRows && !(ringRows && shortTiles) &&
+        (uint64_t)totalVBlocks * tileRows <= kTileMaxReads)
         k_tunnel_v_tile<<<totalVBlocks, 256, (size_t)tileRows * 64 * sizeof(uint32_t), ctx->stream>>>(jobs, nJobs, single,
                                                                                                       seg);
     else if (ringRows)

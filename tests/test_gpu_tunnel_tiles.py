@@ -1,6 +1,6 @@
 """The tunnel's vertical pass in LDS tiles (k_tunnel_v_tile), which launches of
-up to 4096 tiles with segments up to 64 rows take while segment and window fit
-254 rows of LDS: both sides of each of these limits, segments that rows do not
+up to 4096 tiles (fewer of short segments) with segments up to 64 rows take while
+segment and window fit 254 rows of LDS: both sides of each of these limits, segments that rows do not
 divide, columns that tiles do not, windows clipped at either end and at both,
 and a batch of jobs with different windows.  Bit for bit against the oracle."""
 import contextlib
@@ -44,6 +44,15 @@ def test_frame(ctx, orc, W, H, r, seg):
         ctx.tunnel_frame(d, tmp, W, H, ctx.upload(grid), ctx.upload(tex), 9, r)
         got = d.numpy()
     assert np.array_equal(got, _want(orc, W, H, grid, tex, r))
+
+
+# short segments give way to the ring from 1500 tiles on (at 16 rows only below
+# radius 8), the others from 4096 on; past the ring from 860000 rows read on
+@pytest.mark.parametrize("W,H,r,seg", [
+    (1280, 600, 3, 8), (1280, 601, 3, 8), (1280, 1216, 7, 16), (1280, 1216, 8, 16), (1280, 1216, 7, 24),
+    (4096, 2112, 2, 33), (4096, 2113, 2, 33), (1280, 1600, 103, 8), (1280, 1608, 103, 8)])
+def test_limits(ctx, orc, W, H, r, seg):
+    test_frame(ctx, orc, W, H, r, seg)
 
 
 @pytest.mark.parametrize("seg", [16, 32, 64])
