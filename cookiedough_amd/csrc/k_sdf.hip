@@ -655,7 +655,9 @@ __global__ __launch_bounds__(256, kMaxSph > 8 ? 4 : 5) void k_sdf_persistent(uin
 // lane is on the stretch of its ray that can be near any sphere
 // (near_interval): the minimum is the full one to the bit.  The march is VALU
 // bound (a square root and 8 more a sphere and step).  A 1280x720 frame with 8
-// spheres: 65 -> 39 us with the lists and the stretch.
+// spheres: 65 -> 39 us with the lists and the stretch, 34 with a list's spheres four
+// at a time (one at a time past the last eight, as a plain loop has them, 7 spheres
+// of a 320x180 frame took 45 us, 32 now; without lists 33).
 constexpr float kProbe = 1e-3f; // the normal's offset h
 constexpr int kFewSpheres = 6;
 
@@ -719,10 +721,21 @@ __global__ __launch_bounds__(256) void k_sdf(uint32_t *__restrict__ dst, unsigne
             d = hy - sc.groundY;
             if (kFew) {
 #pragma unroll
-                for (int i = 0; i < kFewSpheres; ++i)
-                    if (i < n) d = fminf(d, distance(i, hx, hy, hz));
+                for (int i = 0; i < kFewSpheres; ++i) {
+                    if (i >= n) break;
+                    d = fminf(d, distance(i, hx, hy, hz));
+                }
             } else if (__ballot(total > tNear && total < tFar)) {
-                for (int i = 0; i < n; ++i) d = fminf(d, distance(i, hx, hy, hz));
+                // four at a time, then two and one: a list's latency is its groups'
+                int i = 0;
+                auto next = [&](auto count) {
+#pragma unroll
+                    for (int k = 0; k < decltype(count)::value; ++k) d = fminf(d, distance(i + k, hx, hy, hz));
+                    i += decltype(count)::value;
+                };
+                while (i + 4 <= n) next(std::integral_constant<int, 4>{});
+                if (n & 2) next(std::integral_constant<int, 2>{});
+                if (n & 1) next(std::integral_constant<int, 1>{});
             }
             tHit = total;
             total += d;
@@ -816,11 +829,11 @@ ckd_status launch_sdf(ckd_ctx *ctx, uint32_t *dst, unsigned W, unsigned H,
     const f4 bound = bounding_sphere(sc);
     KernelTimer kt(ctx, CKD_KT_SDF_PLAIN);
     // Frames of few tiles wait for one ray's chain.  All spheres on every step, and
-    // tiles that keep all, against tiles that cull (us): 320x200 with 1 sphere 10.3
-    // / 14.5 / 15.1, 4: 20.6 / 27.1 / 26.7, 8: 34 / 28 / 45, 32: 119 / 84 / 77; 960x540
-    // with 4: 25.7 / 29.2 / 29.0, 8: 49 / 33 / 41, 16: 90 / 55 / 46; 1280x720 with 1:
-    // 17.1 / 18.5 / 19.1, 4: 33.1 / 31.6 / 30.3, 8: 68 / 41 / 42; 2560x1440 with 1: 54 /
-    // 46 / 50, 8: 189 / 87 / 70.
+    // tiles that keep all, against tiles that cull (us): 320x200 with 1 sphere 9.1 /
+    // 13.2 / 13.7, 4: 14.8 / 19.7 / 20.1, 8: - / 29.5 / 31.8, 32: - / 99 / 92; 960x540 with
+    // 4: 21.0 / 22.4 / 23.3, 6: 29.3 / 29.2 / 29.8, 8: - / 31.9 / 33.4, 16: - / 54 / 44;
+    // 1280x720 with 1: 16.0 / 17.1 / 17.4, 4: 32.8 / 25.8 / 25.2, 8: - / 38 / 34; 2560x1440
+    // with 1: 50 / 42 / 46, 8: - / 88 / 71.
     const uint64_t work = (uint64_t)grid.x * grid.y * (unsigned)sc.nSpheres;
     const bool few = sc.nSpheres <= kFewSpheres && work < 10000, cull = work >= 24000 || sc.nSpheres > 16;
     auto launch = [&](auto half, auto fewSpheres) {

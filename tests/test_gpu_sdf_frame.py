@@ -67,3 +67,14 @@ def test_crowd_with_holes(ctx, orc, eps):
         sc.sphere[i][3] = (0.15 + 0.2 * geo[i, 3]) * (-1.0 if i % 8 == 3 else 1.0)
     sc.eps = eps
     _check(ctx, orc, sc, 331, 187, 2.5)
+
+
+@pytest.mark.parametrize("shading", [CKD_SHADE_FP32, CKD_SHADE_FP16])
+@pytest.mark.parametrize("W,H", [(200, 120), (1000, 600)])
+def test_every_length_of_a_list(ctx, orc, W, H, shading):
+    """lists of whole groups of four spheres and every remainder, kept whole (the
+    small frame) and culled"""
+    for n in range(33):
+        sc = wl.sdf_scene(n, max(n, 1), 64)
+        sc.nSpheres = n
+        _check(ctx, orc, sc, W, H, 4.2, shading)
