@@ -98,6 +98,19 @@ def build_shim_test(verbose: bool = True) -> Path:
     return exe
 
 
+def build_test_kernels(verbose: bool = True) -> Path:
+    """The device functions' own test kernels (tests/native/sqrt_sweep.so)."""
+    src = ROOT / "tests" / "native" / "sqrt_sweep.hip"
+    out = src.with_suffix(".so")
+    cmd = [hipcc(), *HIPCC_FLAGS, f"-I{CSRC}", "-shared", str(src), "-o", str(out)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"test kernel build failed:\n{r.stdout}\n{r.stderr}")
+    if verbose:
+        print(f"built {out}")
+    return out
+
+
 def build_oracle(verbose: bool = True) -> None:
     """Compile the oracle (test infrastructure) and, where the reference
     checkout exists, the reference harness oracle/_ref/libckdref.so."""
@@ -116,4 +129,5 @@ def build_oracle(verbose: bool = True) -> None:
 if __name__ == "__main__":
     build()
     build_shim_test()
+    build_test_kernels()
     build_oracle()

@@ -21,6 +21,7 @@
 #include "ckd_internal.h"
 #include "ckd_b07.h"
 #include "ckd_pixel.h"
+#include "ckd_sqrt.h"
 
 #include <cmath>
 #include <cstring>
@@ -112,17 +113,6 @@ struct Lut {
     // lutsinf, ARRESTED_DEV_LEGACY form (code/sincos-lut.h:21-26)
     __device__ __forceinline__ float sin(float a) const { return cos(a + halfPi); }
 };
-
-// sqrtf, correctly rounded: the reciprocal root's product with x and one Newton
-// step on its residual, which the fused multiply-add leaves exact.  It equals
-// sqrtf on every float of the range (compared over all of them); the rest, 0
-// among it, takes sqrtf.  7 instructions instead of 15 of a march step's 125.
-__device__ __forceinline__ float st_sqrt(float x)
-{
-    if (!(x > 0x1p-96f && x < 0x1p96f)) return sqrtf(x);
-    const float y = __builtin_amdgcn_rsqf(x), s = x * y;
-    return fmaf(fmaf(-s, s, x), 0.5f * y, s);
-}
 
 // vFastLen3 of a Vector3 (padding 0): _mm_dp_ps(p, p, 0xff) is
 // (x*x + y*y) + (z*z + 0), and z*z + 0 == z*z for every z
