@@ -190,9 +190,9 @@ CKD_DEV float uniform_f(float v)
 
 // a / b rounded to nearest, from rb = 1 / b rounded to nearest: Markstein's
 // correction of the quotient estimate a * rb (within an ulp) by the residual
-// a - b * (a * rb), which the FMA gives exactly.  For the integers |a| <=
-// 16384 and 1 <= b <= 16384 it equals the IEEE quotient bit for bit (checked
-// over every pair); here |a| <= 4096 and b <= 2160.
+// a - b * (a * rb), which the FMA gives exactly.  For the integers |a| <= 4096 and
+// 1 <= b <= 2160 of a batch it equals the IEEE quotient bit for bit (every pair:
+// tests/test_sdf_setup_arith.py); larger single frames only cull by it.
 CKD_DEV float div_rn(float a, float b, float rb)
 {
     const float q = a * rb;

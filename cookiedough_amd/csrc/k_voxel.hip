@@ -41,10 +41,9 @@ static_assert(sizeof(LsLaunch) + 128 <= 4096, "the kernel's arguments fit 4 KiB"
 // below 2^22: num * rcp(den) is then within 0.5 of num/den, so the estimate
 // floor(num * rcp(den) - 0.5) is the quotient or one less, and one upward
 // correction fixes it.  q*den stays below 2^25, so the 24-bit multiply (full
-// rate; the 32-bit one is quarter rate) is exact.  Checked on the host over
-// every (num, den) of the march with fpFishMul >= 4 (W <= 64 H gives >= 8)
-// and every span divisor, with the reciprocal rounded to nearest and one ulp
-// off either way.
+// rate; the 32-bit one is quarter rate) is exact.  tests/test_voxel_arith.py
+// sweeps it over every span length and every (num, den) of ts_height, with the
+// reciprocal rounded to nearest and one ulp off either way.
 CKD_DEV uint32_t udiv24(uint32_t num, uint32_t den)
 {
     // qf > -0.5: converting through a signed int truncates it to 0 there
@@ -160,9 +159,9 @@ CKD_DEV uint2 ls_span(uint32_t c, uint32_t i, int hgt, int D, int prev)
 // 2^17 as a float; fish >= 8 keeps the quotient below 2^22, so that num *
 // rcp(den) is within 0.5 of num / den, the estimate truncated is the quotient
 // or one less and one upward correction fixes it; the remainder, an integer
-// below 2^18, is exact from one FMA.  Checked on the host over every (num,
-// den) with den = fish * (step + 1) and fish >= 4, the reciprocal rounded to
-// nearest and one ulp off either way.
+// below 2^18, is exact from one FMA.  tests/test_voxel_arith.py sweeps every
+// (num, den) with den = fish * (step + 1) and fish >= 4, the reciprocal rounded
+// to nearest and one ulp off either way.
 CKD_DEV int ls_row(uint32_t h4, uint32_t x, uint32_t y, float denF, uint32_t mapScale, uint32_t tilt8)
 {
     // both lanes fu, then 256 - fu
@@ -474,7 +473,7 @@ constexpr int kTsSteps = (int)kRayLength / 64;
 // = 159 - h) lies within 1/64 of it and its fraction is a multiple of 1/9, so
 // both truncations together are floor(8192 m / (9 n)).  num < 2^21 and den <=
 // 4608: the estimate num * rcp(den) - 0.5 truncated is the quotient or one less
-// (checked on the host over every (m, n)).
+// (tests/test_voxel_arith.py: every (m, n)).
 CKD_DEV int ts_height(uint32_t h, uint32_t n)
 {
     const uint32_t q = udiv24((159u - h) << 13, 9u * n);
