@@ -31,8 +31,9 @@ ckd_status b07_job(uint32_t *img, unsigned W, unsigned H, float strength, B07Job
 // rows, or along the columns with `columns`.  devJobs is the device copy of
 // hostJobs (the host copy picks the kernel and its ring length); vec4: every
 // image 16-byte aligned (rows only).  The kernel is the context tuning's
-// blurKernel: staged lines (lines up to 16383 pixels), a ring per lane, or
-// (0) the ring once the staged lines would need more than one round of blocks.
+// blurKernel: staged lines (lines up to 16383 pixels), a ring per lane, or (0)
+// the scan where its rule takes it, else the ring for columns and once the staged
+// lines would need more than one round of blocks.
 ckd_status blur07_inplace_jobs(ckd_ctx *ctx, const B07Job *hostJobs, const B07Job *devJobs,
                                unsigned n, unsigned W, unsigned H, bool columns, bool vec4,
                                uint32_t *splitStates = nullptr);

@@ -298,9 +298,10 @@ typedef struct ckd_tuning {
                               voxel or tunnel work runs beside the march; a
                               batch of SDF requests only gets at least the
                               kernel's occupancy                            */
-    int tunnelVSeg;        /* rows per lane in the vertical blur: 8..512     */
-    int blurKernel;        /* in-place blur batches: 0 automatic, 1 lines
-                              staged in LDS, 2 an LDS ring per lane          */
+    int tunnelVSeg;        /* rows per segment of the vertical blur: 8..512  */
+    int blurKernel;        /* in-place blur batches: 0 automatic (a scan per
+                              line, or one of these), 1 lines staged in LDS,
+                              2 an LDS ring per lane                         */
     int voxelChunks;       /* 0, 1, 2, 4 or 8 and                           */
     int voxelWavesPerSIMD; /* 0..8: kept for callers that set them; the voxel
                               kernel spreads every march over a block and

@@ -2,9 +2,10 @@
 with pDest == pSrc: the recurrence whose subtract reads already-blurred
 pixels) through ckd_blur07_inplace_batch, and of the Draw calls that use it
 (the ball's blurs and its carried last column, Nautilus, the tunnel's glow),
-with each of its two kernels forced through the tuning: lines staged in LDS
+with each of the two kernels that the tuning can force: lines staged in LDS
 (blurKernel 1) and an LDS ring per lane (blurKernel 2), and the automatic
-choice (0).  Bit-exact against the oracle."""
+choice (0), which at these sizes is mostly the scan.  Bit-exact against the
+oracle."""
 from __future__ import annotations
 
 import contextlib

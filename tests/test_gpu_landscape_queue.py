@@ -1,10 +1,8 @@
-"""ckd_landscape_draw's work queue: a launch whose 64-column groups do not
-spread evenly over the 1024 SIMDs (more than 1024 groups, and at most 90% of
-ceil(groups / 1024) * 1024) splits each column's 512-step march into 2, 4 or
-8 ranges that persistent waves take from a queue, a range waiting for the
-highest row its predecessor drew.  Frames must be bit-identical to the one-wave-per-group
-kernel (voxelChunks 1) and to the oracle (code/landscape.cpp:56-107), for
-every split and queue width, across launches and repeated calls."""
+"""ckd_landscape_draw in calls of many frames, and ckd_tuning's voxelChunks and
+voxelWavesPerSIMD: two fields that once split such calls over a work queue and
+now change nothing (every march is spread over a block).  Frames must equal the
+oracle (code/landscape.cpp:56-107) and be the same for every value that the
+fields take, across launches and repeated calls."""
 import ctypes as C
 
 import numpy as np
@@ -48,9 +46,8 @@ def _oracle(orc, lmaps, W, H, cam):
     return ref
 
 
-# 1280x720 x 60: 1200 groups; 1000x560 x 80: 1280 groups of which the last of
-# each frame is partly outside the row; 640x360 x 200: a 160-frame launch of
-# 1600 groups (queue) and a 40-frame launch of 400 (one wave per group)
+# 1280x720 x 60; 1000x560 x 80: the last block of each frame is partly outside
+# the row; 640x360 x 200: a launch of 160 frames and one of 40
 @pytest.mark.parametrize("W,H,n,check", [(1280, 720, 60, (0, 31, 59)), (1000, 560, 80, (0, 40, 79)),
                                          (640, 360, 200, (0, 159, 160, 199))])
 def test_queue_frames_equal_oracle(ctx, orc, lmaps, W, H, n, check):
@@ -69,8 +66,7 @@ def test_queue_frames_equal_oracle(ctx, orc, lmaps, W, H, n, check):
 
 @pytest.mark.parametrize("waves", [1, 2, 8])
 def test_queue_widths(ctx, orc, lmaps, waves):
-    """1, 2 and 8 persistent waves per SIMD, twice each in a row (the queue
-    and its epoch are reset by the previous launch's last wave)"""
+    """each value of the second field, twice in a row"""
     W, H, n = 1280, 720, 56
     path = wl.landscape_path(1)
     cams = [wl.landscape_cam(path, 0.37 * k) for k in range(n)]
